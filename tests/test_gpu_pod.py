@@ -39,6 +39,40 @@ def test_gram_fp64_parity(m, n, K):
         assert np.array_equal(gs, gs.T)
 
 
+@pytest.mark.parametrize("mode", [pod.GRAM_FP64, pod.GRAM_BF16X3])
+@pytest.mark.parametrize("m,n,K,pad", [(1, 1, 1, 0), (12, 12, 20_001, 1), (16, 5, 4_096, 0),
+                                       (17, 32, 70_003, 0), (33, 48, 9_000, 2), (64, 64, 65_537, 0),
+                                       (64, 49, 300_000, 3)])
+def test_gram_of_few_vectors(mode, m, n, K, pad):
+    """At most 64 vectors: tile edges, K remainders, odd leading dimensions.  FP64 sums in every
+    mode: error at most K eps |X| |Y| entrywise, here far below 1e-13 of the norms' product."""
+    print(f"[case] gram few mode={mode} m={m} n={n} K={K} pad={pad}", flush=True)
+    rng = np.random.default_rng(m + 3 * n)
+    X, Y = rng.standard_normal((m, K)), rng.standard_normal((n, K))
+    Xd, Yd = _dev(np.pad(X, ((0, 0), (0, pad))))[:, :K], _dev(np.pad(Y, ((0, 0), (0, pad))))[:, :K]
+    got = pod.gram(Xd, Yd, mode=mode).cpu().numpy()
+    scale = np.linalg.norm(X, axis=1)[:, None] * np.linalg.norm(Y, axis=1)[None]
+    assert (np.abs(got - X @ Y.T) / scale).max() < 1e-13
+    gs = pod.gram(Xd, mode=mode).cpu().numpy()
+    scale = np.linalg.norm(X, axis=1)
+    assert (np.abs(gs - X @ X.T) / (scale[:, None] * scale[None])).max() < 1e-13
+    assert np.array_equal(gs, gs.T)
+
+
+@pytest.mark.parametrize("m,K", [(65, 5_000), (130, 40_000), (195, 20_011), (384, 50_000)])
+def test_gram_skips_tiles_outside_the_result(m, K):
+    """Blocks cut by the edge of C or by the diagonal, one to a few K slices per block."""
+    print(f"[case] gram tiles m={m} K={K}", flush=True)
+    rng = np.random.default_rng(m)
+    X, Y = rng.standard_normal((m, K)), rng.standard_normal((m, K))
+    scale = np.linalg.norm(X, axis=1)[:, None] * np.linalg.norm(Y, axis=1)[None]
+    full = pod.gram(_dev(X), _dev(Y)).cpu().numpy()
+    assert (np.abs(full - X @ Y.T) / scale).max() < 1e-13
+    gs = pod.gram(_dev(X)).cpu().numpy()
+    assert (np.abs(gs - X @ X.T) / np.linalg.norm(X, axis=1).max() ** 2).max() < 1e-13
+    assert np.array_equal(gs, gs.T)
+
+
 @pytest.mark.parametrize("mode,bound", [(pod.GRAM_FP32X3, 1e-6), (pod.GRAM_BF16X3, 1e-4)])
 def test_gram_split_precision_error(mode, bound):
     rng = np.random.default_rng(1)
