@@ -159,6 +159,176 @@ __global__ void quad_coord3_contract(const double *__restrict__ in,
     y[nQ + g] = fma(df[5 * np + k], x2, fma(df[3 * np + k], x1, df[np + k] * x0));
 }
 
+const char *collapsed_name(const imf_op op)
+{
+    switch (op->shape) {
+    case imf::kSeg: return "segments";
+    case imf::kPyr: return "pyramids";
+    case imf::kTet: return "tetrahedra";
+    case imf::kPrism: return "prisms";
+    default: return "triangles";
+    }
+}
+
+// The runtime-size kernel of a collapsed shape (or segment) on nElmt elements.
+hipError_t launch_general(const imf_op op, bool transpose, int nElmt, int deformed, double lambda,
+                          const double *in, double *out, const double *jac, const double *df,
+                          hipStream_t s)
+{
+    const int geo = op->kind == imf::kBwdTrans ? imf::kUnit : (deformed ? imf::kDeformed : imf::kRegular);
+    auto common = [&](auto &t) {
+        t.kind = op->kind;
+        t.transpose = transpose ? 1 : 0;
+        t.geo = geo;
+        t.nElmt = nElmt;
+        t.tab = op->d_atab;
+        t.in = in;
+        t.out = out;
+        t.jac = jac;
+        t.df = df;
+    };
+    auto directions = [&](auto &t) {
+        common(t);
+        t.nm = op->nmd[0];
+        t.nq0 = op->nqd[0];
+        t.nq1 = op->nqd[1];
+        t.lambda = lambda;
+    };
+    if (op->shape == imf::kSeg) {
+        imf::SegArgs t{};
+        common(t);
+        t.nm = op->nm;
+        t.nq = op->nq;
+        t.ncoord = op->dim;
+        return imf::launch_seg(t, s);
+    }
+    if (op->shape == imf::kTri) {
+        imf::TriArgs t{};
+        directions(t);
+        t.ncoord = op->ncoord == 3 ? 3 : 2;
+        return imf::launch_tri(t, s);
+    }
+    if (op->shape == imf::kPyr) {
+        imf::PyrArgs t{};
+        directions(t);
+        t.nq2 = op->nqd[2];
+        return imf::launch_pyr(t, s);
+    }
+    if (op->shape == imf::kTet) {
+        imf::TetArgs t{};
+        directions(t);
+        t.nq2 = op->nqd[2];
+        return imf::launch_tet(t, s);
+    }
+    imf::PrismArgs t{};
+    directions(t);
+    t.nq2 = op->nqd[2];
+    return imf::launch_prism(t, s);
+}
+
+imf::DenseArgs dense_args(const imf_op op, bool transpose, const double *in, double *out)
+{
+    const int scale = op->deformed ? imf::kScalePoint : imf::kScaleElement;
+    imf::DenseArgs a{};
+    a.sh = op->dense[transpose];
+    a.nElmt = op->nElmt;
+    a.pre = op->kind == imf::kIProduct && !transpose ? scale : imf::kScaleNone;
+    a.post = op->kind == imf::kIProduct && transpose ? scale : imf::kScaleNone;
+    a.lambda = op->lambda;
+    a.tab = op->d_dense[transpose];
+    a.in = in;
+    a.out = out;
+    a.jac = op->d_jac;
+    a.df = op->d_df;
+    return a;
+}
+
+__global__ void fill_identity(int n, double *__restrict__ d)
+{
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < (long)n * n) d[i] = i / n == i % n ? 1.0 : 0.0;
+}
+
+// v[i] = val for i in [0, n), else 0 up to len
+__global__ void fill_range(long len, long lo, long hi, double val, double *__restrict__ d)
+{
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < len) d[i] = i >= lo && i < hi ? val : 0.0;
+}
+
+// The element matrices of a collapsed-shape operator for the dense kernel, read off the
+// runtime-size kernel itself: applied to the identity with unit Jacobians, it gives the
+// matrix with all its vertex and edge corrections.  For Helmholtz the derivative factors are
+// chosen so that one metric term remains: rows e_a give K_aa; a single row e_a + e_b or
+// e_a - e_b gives K_aa + K_bb + (K_ab + K_ba) or the same with a minus sign.
+// Taken by BwdTrans, IProduct and their transposes, and by Helmholtz with one set of factors
+// per element and at most 128 modes.  Time at 12e6 points (at most 120 000 elements), before
+// and now, of 2 / 5 / 8 modes: Helmholtz triangles 250 / 481 / 942 -> 8 / 9 / 41 us,
+// tetrahedra 311 / 950 / 882 -> 9 / 45 / 144 us, prisms of 5 modes 630 -> 133 us; BwdTrans of
+// tetrahedra 67 / 164 / 173 -> 8 / 62 / 94 us, IProduct 78 / 236 / 218 -> 8 / 39 / 98 us.
+int build_dense(imf_op op)
+{
+    const int M = (int)op->M, Q = (int)op->Q;
+    const bool helm = op->kind == imf::kHelmholtz && !op->deformed;
+    if (op->shape == imf::kSeg || !(helm || op->kind == imf::kBwdTrans || op->kind == imf::kIProduct))
+        return IMF_OK;
+    const int D = op->dim, ng = helm ? 1 + D * (D + 1) / 2 : 1;
+    const bool coef_in = op->kind != imf::kIProduct;
+    for (int tr = 0; tr < (helm ? 1 : 2); ++tr) {
+        const bool from_modes = coef_in != (tr == 1);
+        op->dense[tr] = helm ? imf::dense_shape(M, M, ng)
+                             : imf::dense_shape(from_modes ? M : Q, from_modes ? Q : M, 1);
+        // A prism's transform to the points costs its general kernel least (no sums over
+        // shrinking mode ranges): from 30 000 entries on that one is as fast (12e6 points,
+        // 6 / 7 / 8 modes: 99 / 102 / 141 us against 101 / 127 / 165).
+        if (op->shape == imf::kPrism && from_modes && !helm && (long)M * Q > 30000)
+            op->dense[tr].nt = 0;
+    }
+    if (!op->dense[0].nt && !op->dense[1].nt) return IMF_OK;
+    const long n = helm ? M : std::max(M, Q), nd = helm ? (long)D * D * M : 0;
+    double *work = nullptr;
+    hipError_t e = hipMalloc(&work, (size_t)(2 * n * n + n + nd) * sizeof(double));
+    double *eye = work, *mat = eye + n * n, *jac = mat + n * n, *df = jac + n;
+    auto grid = [](long len) { return (unsigned)((len + 255) / 256); };
+    if (e == hipSuccess) fill_range<<<grid(n), 256>>>(n, 0, n, 1.0, jac);
+    for (int tr = 0; tr < 2 && e == hipSuccess; ++tr) {
+        const imf::DenseShape &sh = op->dense[tr];
+        if (!sh.nt) continue;
+        e = hipMalloc(&op->d_dense[tr], sh.tab_len() * sizeof(double));
+        if (e != hipSuccess) break;
+        fill_identity<<<grid((long)sh.K * sh.K), 256>>>(sh.K, eye);
+        // one run of the general kernel on K unit inputs, packed into term g with factor c
+        auto term = [&](int g, double lambda, double c, bool add) {
+            e = launch_general(op, tr == 1, sh.K, 0, lambda, eye, mat, jac, df, nullptr);
+            if (e == hipSuccess) e = imf::dense_pack(sh, g, mat, c, add, op->d_dense[tr], nullptr);
+        };
+        // derivative factors with first row x e_a + y e_b
+        auto factors = [&](int a, double x, int b, double y) {
+            fill_range<<<grid(nd), 256>>>(nd, (long)a * M, (long)(a + 1) * M, x, df);
+            if (b != a) fill_range<<<grid(M), 256>>>(M, 0, M, y, df + (long)b * M);
+        };
+        if (!helm) {
+            term(0, 0.0, 1.0, false);
+            continue;
+        }
+        fill_range<<<grid(nd), 256>>>(nd, 0, 0, 0.0, df);
+        term(0, 1.0, 1.0, false);
+        for (int a = 0, g = 1; a < D; ++a)
+            for (int b = a; b < D && e == hipSuccess; ++b, ++g) {
+                factors(a, 1.0, b, 1.0);
+                term(g, 0.0, a == b ? 1.0 : 0.5, false);
+                if (a == b || e != hipSuccess) continue;
+                factors(a, 1.0, b, -1.0);
+                term(g, 0.0, -0.5, true);
+            }
+    }
+    if (e == hipSuccess) e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    (void)hipFree(work);
+    if (e != hipSuccess) return hip_fail(e, "dense element matrices");
+    return IMF_OK;
+}
+
 int run(imf_op op, imf::LaunchFn fn, const void *in, void *out, void *stream, int nvec = 1,
         long ldin = 0, long ldout = 0, const int *gmap = nullptr,
         const signed char *gsign = nullptr)
@@ -168,106 +338,17 @@ int run(imf_op op, imf::LaunchFn fn, const void *in, void *out, void *stream, in
                                    : needs_df(op) ? "Jacobian and derivative factors not set"
                                                   : "Jacobian not set");
     if (!in || !out) return fail(IMF_ERR_ARG, "null input/output array");
-    if (op->collapsed && op->shape == imf::kSeg) {
-        if (nvec != 1 || gmap) return fail(IMF_ERR_UNSUPPORTED, "segments: one vector per apply");
-        imf::SegArgs t{};
-        t.kind = op->kind;
-        t.transpose = fn == tri_transpose_marker() ? 1 : 0;
-        t.geo = op->kind == imf::kBwdTrans ? imf::kUnit : (op->deformed ? imf::kDeformed : imf::kRegular);
-        t.nm = op->nm;
-        t.nq = op->nq;
-        t.nElmt = op->nElmt;
-        t.ncoord = op->dim;
-        t.tab = op->d_atab;
-        t.in = (const double *)in;
-        t.out = (double *)out;
-        t.jac = op->d_jac;
-        t.df = op->d_df;
-        hipError_t e = imf::launch_seg(t, (hipStream_t)stream);
-        if (e != hipSuccess) return hip_fail(e, "kernel launch");
-        return IMF_OK;
-    }
-    if (op->collapsed && op->shape == imf::kPyr) {
-        if (nvec != 1 || gmap) return fail(IMF_ERR_UNSUPPORTED, "pyramids: one vector per apply");
-        imf::PyrArgs t{};
-        t.kind = op->kind;
-        t.transpose = fn == tri_transpose_marker() ? 1 : 0;
-        t.geo = op->kind == imf::kBwdTrans ? imf::kUnit : (op->deformed ? imf::kDeformed : imf::kRegular);
-        t.nm = op->nmd[0];
-        t.nq0 = op->nqd[0];
-        t.nq1 = op->nqd[1];
-        t.nq2 = op->nqd[2];
-        t.nElmt = op->nElmt;
-        t.lambda = op->lambda;
-        t.tab = op->d_atab;
-        t.in = (const double *)in;
-        t.out = (double *)out;
-        t.jac = op->d_jac;
-        t.df = op->d_df;
-        hipError_t e = imf::launch_pyr(t, (hipStream_t)stream);
-        if (e != hipSuccess) return hip_fail(e, "kernel launch");
-        return IMF_OK;
-    }
-    if (op->collapsed && op->shape == imf::kTet) {
-        if (nvec != 1 || gmap) return fail(IMF_ERR_UNSUPPORTED, "tetrahedra: one vector per apply");
-        imf::TetArgs t{};
-        t.kind = op->kind;
-        t.transpose = fn == tri_transpose_marker() ? 1 : 0;
-        t.geo = op->kind == imf::kBwdTrans ? imf::kUnit : (op->deformed ? imf::kDeformed : imf::kRegular);
-        t.nm = op->nmd[0];
-        t.nq0 = op->nqd[0];
-        t.nq1 = op->nqd[1];
-        t.nq2 = op->nqd[2];
-        t.nElmt = op->nElmt;
-        t.lambda = op->lambda;
-        t.tab = op->d_atab;
-        t.in = (const double *)in;
-        t.out = (double *)out;
-        t.jac = op->d_jac;
-        t.df = op->d_df;
-        hipError_t e = imf::launch_tet(t, (hipStream_t)stream);
-        if (e != hipSuccess) return hip_fail(e, "kernel launch");
-        return IMF_OK;
-    }
-    if (op->collapsed && op->shape == imf::kPrism) {
-        if (nvec != 1 || gmap) return fail(IMF_ERR_UNSUPPORTED, "prisms: one vector per apply");
-        imf::PrismArgs t{};
-        t.kind = op->kind;
-        t.transpose = fn == tri_transpose_marker() ? 1 : 0;
-        t.geo = op->kind == imf::kBwdTrans ? imf::kUnit : (op->deformed ? imf::kDeformed : imf::kRegular);
-        t.nm = op->nmd[0];
-        t.nq0 = op->nqd[0];
-        t.nq1 = op->nqd[1];
-        t.nq2 = op->nqd[2];
-        t.nElmt = op->nElmt;
-        t.lambda = op->lambda;
-        t.tab = op->d_atab;
-        t.in = (const double *)in;
-        t.out = (double *)out;
-        t.jac = op->d_jac;
-        t.df = op->d_df;
-        hipError_t e = imf::launch_prism(t, (hipStream_t)stream);
-        if (e != hipSuccess) return hip_fail(e, "kernel launch");
-        return IMF_OK;
-    }
     if (op->collapsed) {
-        if (nvec != 1 || gmap) return fail(IMF_ERR_UNSUPPORTED, "triangles: one vector per apply");
-        imf::TriArgs t{};
-        t.kind = op->kind;
-        t.transpose = fn == tri_transpose_marker() ? 1 : 0;
-        t.geo = op->kind == imf::kBwdTrans ? imf::kUnit : (op->deformed ? imf::kDeformed : imf::kRegular);
-        t.nm = op->nmd[0];
-        t.nq0 = op->nqd[0];
-        t.nq1 = op->nqd[1];
-        t.nElmt = op->nElmt;
-        t.ncoord = op->ncoord == 3 ? 3 : 2;
-        t.lambda = op->lambda;
-        t.tab = op->d_atab;
-        t.in = (const double *)in;
-        t.out = (double *)out;
-        t.jac = op->d_jac;
-        t.df = op->d_df;
-        hipError_t e = imf::launch_tri(t, (hipStream_t)stream);
+        if (nvec != 1 || gmap)
+            return fail(IMF_ERR_UNSUPPORTED, std::string(collapsed_name(op)) + ": one vector per apply");
+        const bool tr = fn == tri_transpose_marker();
+        hipError_t e;
+        if (op->d_dense[tr])
+            e = imf::launch_dense(dense_args(op, tr, (const double *)in, (double *)out),
+                                  (hipStream_t)stream);
+        else
+            e = launch_general(op, tr, op->nElmt, op->deformed, op->lambda, (const double *)in,
+                               (double *)out, op->d_jac, op->d_df, (hipStream_t)stream);
         if (e != hipSuccess) return hip_fail(e, "kernel launch");
         return IMF_OK;
     }
@@ -809,16 +890,17 @@ int imf_create(const char *key, int dim, const int *nm, const int *nq,
         if (precision != IMF_FP64 && precision != IMF_FP32)
             return fail(IMF_ERR_ARG, "imf_create: unknown precision");
         if (nElmt <= 0) return fail(IMF_ERR_ARG, "imf_create: nElmt must be positive");
-        if (shape == imf::kPyr)
-            return create_pyr(k, kind, deformed, nm, nq, bdata, dbdata, D, w, nElmt, precision,
-                              out);
-        if (shape == imf::kTet)
-            return create_tet(k, kind, deformed, nm, nq, bdata, dbdata, D, w, nElmt, precision,
-                              out);
-        if (shape == imf::kPrism)
-            return create_prism(k, kind, deformed, nm, nq, bdata, dbdata, D, w, nElmt, precision,
-                                out);
-        return create_tri(k, kind, deformed, nm, nq, bdata, dbdata, D, w, nElmt, precision, out);
+        const auto create = shape == imf::kPyr ? create_pyr : shape == imf::kTet ? create_tet
+                          : shape == imf::kPrism ? create_prism : create_tri;
+        imf_op op = nullptr;
+        if (int st = create(k, kind, deformed, nm, nq, bdata, dbdata, D, w, nElmt, precision, &op))
+            return st;
+        if (int st = build_dense(op)) {
+            imf_destroy(op);
+            return st;
+        }
+        *out = op;
+        return IMF_OK;
     }
     if (dim != shape)
         return fail(IMF_ERR_ARG, "imf_create: dim does not match the shape of " + k);
@@ -891,6 +973,8 @@ int imf_destroy(imf_op op)
     (void)hipFree(op->d_in);
     (void)hipFree(op->d_out);
     (void)hipFree(op->d_atab);
+    (void)hipFree(op->d_dense[0]);
+    (void)hipFree(op->d_dense[1]);
     for (int b = 0; b < 2; ++b) {
         (void)hipHostFree(op->pin_in[b]);
         (void)hipHostFree(op->pin_out[b]);

@@ -6,6 +6,7 @@
 
 #include "imf_common.hpp"
 #include "mf_aniso.hpp"
+#include "mf_dense.hpp"
 #include "mf_prism.hpp"
 #include "mf_pyr.hpp"
 #include "mf_tet.hpp"
@@ -49,6 +50,9 @@ struct imf_op_s {
     // (mf_tet.hip) and pyramids (mf_pyr.hip; nqd[0..2] along eta0 / eta1 / eta2), nmd[0]
     // modes per direction, the table image in d_atab; geometry read unpacked from d_jac / d_df
     bool collapsed = false;
+    // forward / transpose as dense products over the elements (mf_dense.hip), when built
+    imf::DenseShape dense[2];
+    double *d_dense[2] = {nullptr, nullptr};
 };
 
 // Kernel arguments of an anisotropic operator's apply (in, out, nvec vectors at ld strides).

@@ -1,0 +1,78 @@
+"""Operators of the collapsed shapes at the sizes where their kernels' tiles end (one element,
+one less and one more than a tile of 16, one more than a workgroup's 64; 2 to 8 modes, so
+1 to 18 column tiles), against the CPU oracle.  Bar: 1e-12 relative, as for the operators'
+other parity tests (about 1e3 roundings of 1e-16 with condition 10)."""
+import numpy as np
+import pytest
+import torch
+
+import ithaca_hip as H
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+REG = {"tri": [[0, 0], [1, 0], [0, 1]],
+       "tet": [[0, 0, 0], [1, 0, 0], [0, 1, 0], [0, 0, 1]],
+       "prism": [[0, 0, 0], [1, 0, 0], [1, 1, 0], [0, 1, 0], [0.5, 0, 1], [0.5, 1, 1]],
+       "pyr": [[0, 0, 0], [1, 0, 0], [1, 1, 0], [0, 1, 0], [0.5, 0.5, 0.9]]}
+
+
+def _basis(shape, nm, nq):
+    if shape == "tri":
+        return O.basis_tri(nm, nq)
+    if shape == "tet":
+        return O.basis_tet(nm, nq, nq - 1, nq - 1)
+    return getattr(O, f"basis_{shape}")(nm, nq, nq - 1)
+
+
+def _tables(shape, b):
+    raw = {"tri": [1], "tet": [1, 2], "prism": [2], "pyr": [2]}[shape]
+    return [dict(bdata=b[f"bdata{d}"], dbdata=b[f"dbdata{d}"], D=b[f"D{d}"],
+                 w=b[f"w{d}_raw"] if d in raw else b[f"w{d}"]) for d in range(2 if shape == "tri" else 3)]
+
+
+def _rel(a, r):
+    return np.linalg.norm(a - r) / np.linalg.norm(r)
+
+
+@pytest.mark.parametrize("E", [1, 15, 17, 65])
+@pytest.mark.parametrize("nm,extra", [(2, 1), (3, 2), (5, 1), (6, 2), (8, 1)])
+@pytest.mark.parametrize("deformed", [False, True])
+@pytest.mark.parametrize("shape", ["tri", "tet", "prism", "pyr"])
+def test_element_counts_and_orders(shape, deformed, nm, extra, E):
+    print(f"[case] {shape} nm={nm} nq=+{extra} E={E} deformed={deformed}", flush=True)
+    nq = nm + extra
+    rng = np.random.default_rng(E + nm)
+    R = np.array(REG[shape], dtype=float)
+    jitter = 0.1 if deformed or shape in ("tri", "tet") else 0.0
+    verts = np.stack([R * rng.uniform(0.5, 2.0) + jitter * rng.uniform(-1, 1, R.shape) for _ in range(E)])
+    b = _basis(shape, nm, nq)
+    jac, df = getattr(O, f"geom_{shape}")(verts, b, deformed)
+    geo, cap = "Deformed" if deformed else "Regular", shape.capitalize()
+    u, f = rng.uniform(-1, 1, E * b["M"]), rng.uniform(-1, 1, E * b["Q"])
+    du, dfq = torch.from_numpy(u).cuda(), torch.from_numpy(f).cuda()
+
+    def op(kind, g=geo):
+        o = H.Operator(f"{kind}_{cap}_{g}", nm, tuple(b[f"nq{d}"] for d in range(R.shape[1])), E,
+                       basis=_tables(shape, b))
+        if o.needs_jac():
+            o.set_jac(jac)
+        if o.needs_df():
+            o.set_df(df)
+        return o
+
+    bw, ip, hm = op("BwdTrans", "Regular"), op("IProduct"), op("Helmholtz")
+    hm.set_lambda(2.5)
+    Bu = getattr(O, f"bwdtrans_{shape}")(b, E, u)
+    Pf = getattr(O, f"iproduct_{shape}")(b, E, deformed, jac, f)
+    assert _rel(bw.apply(du).cpu().numpy(), Bu) < 1e-12
+    assert _rel(ip.apply(dfq).cpu().numpy(), Pf) < 1e-12
+    assert _rel(hm.apply(du).cpu().numpy(),
+                getattr(O, f"helmholtz_{shape}")(b, E, deformed, jac, df, 2.5, u)) < 1e-12
+    # transposes by their definition, element by element
+    by = lambda a, n: a.reshape(E, n)
+    Bt = bw.apply_transpose(dfq).cpu().numpy()
+    Pt = ip.apply_transpose(du).cpu().numpy()
+    scale = np.linalg.norm(u) * np.linalg.norm(f)
+    assert np.abs((by(Bt, b["M"]) * by(u, b["M"])).sum(1) - (by(Bu, b["Q"]) * by(f, b["Q"])).sum(1)).max() < 1e-12 * scale
+    assert np.abs((by(Pt, b["Q"]) * by(f, b["Q"])).sum(1) - (by(Pf, b["M"]) * by(u, b["M"])).sum(1)).max() < 1e-12 * scale
