@@ -6,6 +6,7 @@
 // image.  Applies on device arrays allocate nothing.
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <condition_variable>
 #include <cstdio>
 #include <cstring>
@@ -74,6 +75,26 @@ int maybe_pack(imf_op op)
     if (needs_jac(op) && !op->d_jac) return IMF_OK;
     if (needs_df(op) && !op->d_df) return IMF_OK;
     if (op->aniso || op->collapsed) {  // these kernels read GetJac / GetDerivFactors directly
+        if (op->pencil[0] && op->kind == imf::kHelmholtz && op->deformed) {  // packed for them
+            const int *q = op->nqd;
+            const long len = (long)op->nElmt * imf::geo_stride(7l * op->Q, 8);
+            hipError_t e = hipSuccess;
+            if (!op->d_geom) e = hipMalloc(&op->d_geom, len * sizeof(double));
+            const double *w[3];
+            size_t off = 0;
+            const int m = op->nmd[0], tri = imf::tri_modes(m);
+            const int rows[3] = {m, op->shape == imf::kTet ? tri : m,
+                                 op->shape == imf::kPrism ? tri : (int)op->M};
+            for (int d = 0; d < 3; ++d) {  // B dB D w z of each direction
+                off += 2 * (size_t)rows[d] * q[d] + (size_t)q[d] * q[d];
+                w[d] = op->d_atab + off;
+                off += 2 * (size_t)q[d];
+            }
+            if (e == hipSuccess)
+                e = imf::pencil_pack(op->nElmt, q, w, op->d_jac, op->d_df, (double *)op->d_geom, nullptr);
+            if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+            if (e != hipSuccess) return hip_fail(e, "packed geometry");
+        }
         static std::atomic<unsigned long> next_id{1ul << 62};
         op->geom_ready = true;
         op->geom_version = next_id.fetch_add(1);
@@ -256,16 +277,87 @@ __global__ void fill_range(long len, long lo, long hi, double val, double *__res
     if (i < len) d[i] = i >= lo && i < hi ? val : 0.0;
 }
 
+imf::PencilArgs pencil_args(const imf_op op, const double *in, double *out)
+{
+    imf::PencilArgs a{};
+    a.nElmt = op->nElmt;
+    a.scaled = op->kind == imf::kIProduct ? 1 : 0;
+    a.deformed = op->deformed;
+    a.lambda = op->lambda;
+    a.tab = op->d_atab;
+    a.in = in;
+    a.out = out;
+    a.jac = op->d_jac;
+    a.df = op->d_df;
+    a.geom = (const double *)op->d_geom;
+    return a;
+}
+
+// Pencil kernels of a prism, tetrahedron or pyramid operator: sizes they are compiled for,
+// and tables with dbdata = D bdata (to rounding), which lets the kernels apply D^T instead of
+// separate inner products with dbdata.
+void find_pencil(imf_op op, const double *const *bdata, const double *const *dbdata,
+                 const double *const *D)
+{
+    if (op->shape != imf::kPrism && op->shape != imf::kTet && op->shape != imf::kPyr) return;
+    const int m = op->nmd[0], q0 = op->nqd[0];
+    const bool tet = op->shape == imf::kTet;
+    if (op->nqd[1] != (tet ? q0 - 1 : q0) || op->nqd[2] != q0 - 1) return;
+    const auto lookup = op->shape == imf::kPrism ? imf::lookup_pencil_prism
+                      : tet ? imf::lookup_pencil_tet : imf::lookup_pencil_pyr;
+    if (op->kind == imf::kHelmholtz || op->kind == imf::kIProdDeriv) {
+        const int tri = imf::tri_modes(m);
+        const int rows[3] = {m, tet ? tri : m, op->shape == imf::kPrism ? tri : (int)op->M};
+        for (int d = 0; d < 3; ++d) {
+            const int q = op->nqd[d];
+            double big = 0.0, off = 0.0;
+            for (int r = 0; r < rows[d]; ++r)
+                for (int i = 0; i < q; ++i) {
+                    double s = 0.0;
+                    for (int a = 0; a < q; ++a) s += bdata[d][r * q + a] * D[d][a * q + i];
+                    big = std::max(big, std::fabs(dbdata[d][r * q + i]));
+                    off = std::max(off, std::fabs(s - dbdata[d][r * q + i]));
+                }
+            if (!(off <= 1e-12 * big)) return;
+        }
+    }
+    const bool swap = op->kind == imf::kBwdTrans || op->kind == imf::kIProduct;
+    op->pencil[0] = lookup(op->kind, m, q0);
+    if (swap)
+        op->pencil[1] = lookup(op->kind == imf::kBwdTrans ? imf::kIProduct : imf::kBwdTrans, m, q0);
+}
+
+// Dense products against the other kernels.  A dense product costs its matrix's entries per
+// element, a pencil kernel about the number of points.  Times in us at 12e6 points (at most
+// 120 000 elements), one point more than modes, dense / pencils, of 2 3 4 5 6 7 8 modes:
+//   Helmholtz  tetrahedra   9/20  14/48  31/98  45/152  48/177  72/207  144/242
+//              prisms       9/23  30/47  67/96  133/97  222/109  -/149  -/149
+//              pyramids     9/23  14/47  38/103 73/104  114/115  -/157  -/206
+//     (two points more: prisms of 5 and 6 modes 83/100, 150/133; pyramids of 6 80/112)
+//   BwdTrans   tetrahedra   9/8   16/20  27/33  51/53   52/50    78/66  101/69
+//              prisms      12/9   17/21  56/36  77/45  101/44   127/53  165/57
+//              pyramids    12/9   17/19  39/36  60/46   79/45   108/63  139/76
+//   IProduct   tetrahedra   8/9   13/25  28/54  39/79   41/74   57/106   97/109
+//              prisms       8/12  20/24  43/47  58/61  100/59   137/72  163/74
+//              pyramids     8/12  14/24  35/49  50/64   80/65   103/106 160/116
+// Without a pencil kernel (triangles, other point counts) the alternative is the runtime-size
+// kernel, which only a prism's transform to the points with 30 000 entries or more meets
+// (6 / 7 / 8 modes: 99 / 102 / 141 us).
+bool dense_pays(const imf_op op, int tr, bool helm, bool from_modes)
+{
+    const long M = (long)op->M, Q = (long)op->Q;
+    if (!op->pencil[tr]) return helm || !from_modes || op->shape != imf::kPrism || M * Q <= 30000;
+    if (helm) return M * M < 27 * Q;
+    return from_modes ? M <= 20 : op->shape == imf::kTet || M <= 80;
+}
+
 // The element matrices of a collapsed-shape operator for the dense kernel, read off the
 // runtime-size kernel itself: applied to the identity with unit Jacobians, it gives the
 // matrix with all its vertex and edge corrections.  For Helmholtz the derivative factors are
 // chosen so that one metric term remains: rows e_a give K_aa; a single row e_a + e_b or
 // e_a - e_b gives K_aa + K_bb + (K_ab + K_ba) or the same with a minus sign.
-// Taken by BwdTrans, IProduct and their transposes, and by Helmholtz with one set of factors
-// per element and at most 128 modes.  Time at 12e6 points (at most 120 000 elements), before
-// and now, of 2 / 5 / 8 modes: Helmholtz triangles 250 / 481 / 942 -> 8 / 9 / 41 us,
-// tetrahedra 311 / 950 / 882 -> 9 / 45 / 144 us, prisms of 5 modes 630 -> 133 us; BwdTrans of
-// tetrahedra 67 / 164 / 173 -> 8 / 62 / 94 us, IProduct 78 / 236 / 218 -> 8 / 39 / 98 us.
+// Taken by BwdTrans, IProduct and their transposes and by Helmholtz with one set of factors
+// per element and at most 128 modes, where dense_pays().
 int build_dense(imf_op op)
 {
     const int M = (int)op->M, Q = (int)op->Q;
@@ -278,11 +370,7 @@ int build_dense(imf_op op)
         const bool from_modes = coef_in != (tr == 1);
         op->dense[tr] = helm ? imf::dense_shape(M, M, ng)
                              : imf::dense_shape(from_modes ? M : Q, from_modes ? Q : M, 1);
-        // A prism's transform to the points costs its general kernel least (no sums over
-        // shrinking mode ranges): from 30 000 entries on that one is as fast (12e6 points,
-        // 6 / 7 / 8 modes: 99 / 102 / 141 us against 101 / 127 / 165).
-        if (op->shape == imf::kPrism && from_modes && !helm && (long)M * Q > 30000)
-            op->dense[tr].nt = 0;
+        if (!dense_pays(op, tr, helm, from_modes)) op->dense[tr].nt = 0;
     }
     if (!op->dense[0].nt && !op->dense[1].nt) return IMF_OK;
     const long n = helm ? M : std::max(M, Q), nd = helm ? (long)D * D * M : 0;
@@ -346,6 +434,9 @@ int run(imf_op op, imf::LaunchFn fn, const void *in, void *out, void *stream, in
         if (op->d_dense[tr])
             e = imf::launch_dense(dense_args(op, tr, (const double *)in, (double *)out),
                                   (hipStream_t)stream);
+        else if (op->pencil[tr])
+            e = op->pencil[tr](pencil_args(op, (const double *)in, (double *)out),
+                               (hipStream_t)stream);
         else
             e = launch_general(op, tr, op->nElmt, op->deformed, op->lambda, (const double *)in,
                                (double *)out, op->d_jac, op->d_df, (hipStream_t)stream);
@@ -546,6 +637,16 @@ int create_tri(const std::string &k, int kind, int deformed, const int *nm, cons
     return IMF_OK;
 }
 
+// The collapse factors the pencil kernels read after the image (pencil_extra doubles).
+void append_collapse(std::vector<double> &tab, const std::vector<double> &z0,
+                     const std::vector<double> &z1, const std::vector<double> &z2)
+{
+    for (double z : z0) tab.push_back(0.5 * (1.0 + z));
+    for (double z : z1) tab.push_back(0.5 * (1.0 + z));
+    for (double z : z1) tab.push_back(z < 1.0 ? 2.0 / (1.0 - z) : 0.0);  // tetrahedra only
+    for (double z : z2) tab.push_back(2.0 / (1.0 - z));
+}
+
 // Prisms: Modified_A x Modified_A x Modified_B in collapsed coordinates (mf_prism.hip),
 // FP64.  Directions 0 and 1: bdata/dbdata nm*nq[d], D nq[d]^2, w nq[d] (GLL); direction 2:
 // bdata/dbdata nm(nm+1)/2 * nq[2], D nq[2]^2, w nq[2] (the Gauss-Radau alpha = 1 weights;
@@ -609,6 +710,7 @@ int create_prism(const std::string &k, int kind, int deformed, const int *nm, co
     put(D[2], (size_t)q2 * q2);
     for (int j = 0; j < q2; ++j) tab.push_back(0.5 * w[2][j]);
     put(z2.data(), q2);
+    append_collapse(tab, z0, z1, z2);
     imf_op op = new imf_op_s();
     op->kind = kind; op->shape = imf::kPrism; op->deformed = deformed; op->prec = precision;
     op->dim = 3; op->nm = m; op->nq = q0; op->nElmt = nElmt;
@@ -690,6 +792,7 @@ int create_tet(const std::string &k, int kind, int deformed, const int *nm, cons
         for (int j = 0; j < qd[d]; ++j) tab.push_back(fac[d] * w[d][j]);
         put(zd[d], qd[d]);
     }
+    append_collapse(tab, z0, z1, z2);
     imf_op op = new imf_op_s();
     op->kind = kind; op->shape = imf::kTet; op->deformed = deformed; op->prec = precision;
     op->dim = 3; op->nm = m; op->nq = q0; op->nElmt = nElmt;
@@ -771,6 +874,7 @@ int create_pyr(const std::string &k, int kind, int deformed, const int *nm, cons
         for (int j = 0; j < qd[d]; ++j) tab.push_back(fac[d] * w[d][j]);
         put(zd[d], qd[d]);
     }
+    append_collapse(tab, z0, z1, z2);
     imf_op op = new imf_op_s();
     op->kind = kind; op->shape = imf::kPyr; op->deformed = deformed; op->prec = precision;
     op->dim = 3; op->nm = m; op->nq = q0; op->nElmt = nElmt;
@@ -895,6 +999,7 @@ int imf_create(const char *key, int dim, const int *nm, const int *nq,
         imf_op op = nullptr;
         if (int st = create(k, kind, deformed, nm, nq, bdata, dbdata, D, w, nElmt, precision, &op))
             return st;
+        find_pencil(op, bdata, dbdata, D);
         if (int st = build_dense(op)) {
             imf_destroy(op);
             return st;

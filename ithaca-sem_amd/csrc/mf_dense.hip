@@ -141,7 +141,7 @@ __global__ __launch_bounds__(256) void dense_kernel(DenseArgs a)
             if (n >= N) continue;
             double v = acc[t][r] * jo;
             if (a.post == kScalePoint) v *= a.jac[er * N + n];
-            __builtin_nontemporal_store(v, a.out + er * N + n);
+            a.out[er * N + n] = v;
         }
     }
 }

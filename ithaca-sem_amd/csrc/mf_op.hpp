@@ -7,6 +7,7 @@
 #include "imf_common.hpp"
 #include "mf_aniso.hpp"
 #include "mf_dense.hpp"
+#include "mf_pencil.hpp"
 #include "mf_prism.hpp"
 #include "mf_pyr.hpp"
 #include "mf_tet.hpp"
@@ -53,6 +54,8 @@ struct imf_op_s {
     // forward / transpose as dense products over the elements (mf_dense.hip), when built
     imf::DenseShape dense[2];
     double *d_dense[2] = {nullptr, nullptr};
+    // forward / transpose pencil kernels (mf_pencil_kernels.hpp), for the orders they cover
+    imf::PencilFn pencil[2] = {nullptr, nullptr};
 };
 
 // Kernel arguments of an anisotropic operator's apply (in, out, nvec vectors at ld strides).

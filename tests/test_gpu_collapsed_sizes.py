@@ -62,6 +62,12 @@ def test_element_counts_and_orders(shape, deformed, nm, extra, E):
         return o
 
     bw, ip, hm = op("BwdTrans", "Regular"), op("IProduct"), op("Helmholtz")
+    dim = R.shape[1]
+    pd = op("PhysDeriv").apply(dfq).cpu().numpy()
+    assert _rel(pd, np.concatenate(getattr(O, f"physderiv_{shape}")(b, E, deformed, df, f))) < 1e-12
+    v = rng.uniform(-1, 1, (dim, E * b["Q"]))
+    assert _rel(op("IProductWRTDerivBase").apply(torch.from_numpy(v.reshape(-1)).cuda()).cpu().numpy(),
+                getattr(O, f"iprodderiv_{shape}")(b, E, deformed, jac, df, *([*v] if dim == 2 else [v]))) < 1e-12
     hm.set_lambda(2.5)
     Bu = getattr(O, f"bwdtrans_{shape}")(b, E, u)
     Pf = getattr(O, f"iproduct_{shape}")(b, E, deformed, jac, f)
@@ -76,3 +82,26 @@ def test_element_counts_and_orders(shape, deformed, nm, extra, E):
     scale = np.linalg.norm(u) * np.linalg.norm(f)
     assert np.abs((by(Bt, b["M"]) * by(u, b["M"])).sum(1) - (by(Bu, b["Q"]) * by(f, b["Q"])).sum(1)).max() < 1e-12 * scale
     assert np.abs((by(Pt, b["Q"]) * by(f, b["Q"])).sum(1) - (by(Pf, b["M"]) * by(u, b["M"])).sum(1)).max() < 1e-12 * scale
+
+
+@pytest.mark.parametrize("shape", ["prism", "tet", "pyr"])
+def test_dbdata_that_is_not_d_bdata_is_still_used(shape):
+    """The kernels that apply D^T in place of dbdata only take tables where the two agree: with
+    dbdata doubled, the stiffness part (lambda = 0) is exactly twice as large."""
+    nm, E = 4, 9
+    rng = np.random.default_rng(3)
+    R = np.array(REG[shape], dtype=float)
+    verts = np.stack([R + 0.1 * rng.uniform(-1, 1, R.shape) for _ in range(E)])
+    b = _basis(shape, nm, nm + 1)
+    jac, df = getattr(O, f"geom_{shape}")(verts, b, True)
+    u = torch.from_numpy(rng.uniform(-1, 1, E * b["M"])).cuda()
+    got = []
+    for c in (1.0, 2.0):
+        tabs = [dict(t, dbdata=c * t["dbdata"]) for t in _tables(shape, b)]
+        o = H.Operator(f"Helmholtz_{shape.capitalize()}_Deformed", nm, tuple(b[f"nq{d}"] for d in range(3)),
+                       E, basis=tabs)
+        o.set_jac(jac)
+        o.set_df(df)
+        o.set_lambda(0.0)
+        got.append(o.apply(u).cpu().numpy())
+    assert _rel(got[1], 2.0 * got[0]) < 1e-12
