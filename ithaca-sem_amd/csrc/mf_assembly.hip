@@ -371,29 +371,33 @@ __global__ void g2l_kernel(long n, const int *__restrict__ l2g, const signed cha
 }
 
 // global[g] = sum over the local modes mapped to g of sign * local (Vmath::Assmb), as a
-// deterministic gather over the inverse map (CSR: off[g]..off[g+1] into inv).
-// With sg == NULL the contributions are added unsigned (the assembled diagonal:
+// deterministic gather over the inverse map (CSR: off[g]..off[g+1] into inv; an entry is the
+// local index with the sign in its top bit, which saves the gather of a separate sign byte
+// per copy).  kUnsigned adds the contributions without signs (the assembled diagonal:
 // sign^2 = 1).
+template <bool kUnsigned>
 __device__ __forceinline__ double assemble_one(long g, const int *__restrict__ off,
-                                               const int *__restrict__ inv,
-                                               const signed char *__restrict__ sg,
+                                               const unsigned *__restrict__ inv,
                                                const double *__restrict__ loc,
                                                const unsigned char *__restrict__ mask)
 {
     double s = 0.0;
-    for (int k = off[g]; k < off[g + 1]; ++k) {
-        const int i = inv[k];
-        s += sg ? sg[i] * loc[i] : loc[i];
+    const int k1 = off[g + 1];
+    for (int k = off[g]; k < k1; ++k) {
+        const unsigned i = inv[k];
+        const double v = loc[i & 0x7fffffffu];
+        s += !kUnsigned && (i >> 31) ? -v : v;
     }
     return (mask && mask[g]) ? 0.0 : s;
 }
 
-__global__ void assemble_kernel(long ng, const int *__restrict__ off, const int *__restrict__ inv,
-                                const signed char *__restrict__ sg, const double *__restrict__ loc,
+template <bool kUnsigned>
+__global__ void assemble_kernel(long ng, const int *__restrict__ off, const unsigned *__restrict__ inv,
+                                const double *__restrict__ loc,
                                 const unsigned char *__restrict__ mask, double *__restrict__ glob)
 {
     const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g < ng) glob[g] = assemble_one(g, off, inv, sg, loc, mask);
+    if (g < ng) glob[g] = assemble_one<kUnsigned>(g, off, inv, loc, mask);
 }
 
 __global__ void zero_kernel(long n, double *__restrict__ x)
@@ -408,36 +412,67 @@ struct DiagTab {
 
 // Local diagonal of the Helmholtz operator lambda M + sum_ab (D_a B)^T diag(w J G^ab) (D_b B)
 // from the operator's packed geometry (deformed [e][GS], GS = 7Q rounded to 128-byte lines;
-// regular [e][7] with the weights applied here); one thread per (element, mode).
-__global__ void helm_diag_hex(DiagTab t, int nm, int nq, long nElmt, int deformed, double lambda,
-                              const double *__restrict__ geom, double *__restrict__ diag)
+// regular [e][7] with the weights applied here).  One workgroup per element: the diagonal is a
+// sum over the seven geometry terms of separable weights (B^2, dB^2 or B dB per direction), so
+// each term is contracted one direction at a time through LDS.  With one thread per mode
+// summing over all points it read the geometry once per mode (8 000 elements of 6 modes:
+// 2.5 ms; now 0.2 ms).
+__global__ __launch_bounds__(256) void helm_diag_hex(DiagTab t, int nm, int nq, int deformed,
+                                                     double lambda,
+                                                     const double *__restrict__ geom,
+                                                     double *__restrict__ diag)
 {
-    const long M = (long)nm * nm * nm, Q = (long)nq * nq * nq;
-    const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= nElmt * M) return;
-    const long e = g / M;
-    const int md = (int)(g - e * M), p = md % nm, q = (md / nm) % nm, r = md / (nm * nm);
-    const long GS = imf::geo_stride(7 * Q, sizeof(double));
-    double s = 0.0;
-    for (int k = 0; k < nq; ++k)
-        for (int j = 0; j < nq; ++j)
-            for (int i = 0; i < nq; ++i) {
-                const long pt = ((long)k * nq + j) * nq + i;
-                const double bp = t.B[p * nq + i], bq = t.B[q * nq + j], br = t.B[r * nq + k];
-                const double phi = bp * bq * br;
-                const double d0 = t.dB[p * nq + i] * bq * br, d1 = bp * t.dB[q * nq + j] * br,
-                             d2 = bp * bq * t.dB[r * nq + k];
-                double c[7];
-                if (deformed) {
-                    for (int a = 0; a < 7; ++a) c[a] = geom[e * GS + a * Q + pt];
-                } else {
-                    const double wq = t.w[i] * t.w[j] * t.w[k];
-                    for (int a = 0; a < 7; ++a) c[a] = geom[e * 7 + a] * wq;
-                }
-                s += lambda * c[0] * phi * phi + c[1] * d0 * d0 + c[4] * d1 * d1 + c[6] * d2 * d2 +
-                     2.0 * (c[2] * d0 * d1 + c[3] * d0 * d2 + c[5] * d1 * d2);
-            }
-    diag[g] = s;
+    extern __shared__ double sm[];
+    const int M = nm * nm * nm, Q = nq * nq * nq, n1 = nq * nq * nm, n2 = nq * nm * nm;
+    // squares and products of the tables, then the point array and two partial contractions
+    double *T0 = sm, *T1 = T0 + nm * nq, *T2 = T1 + nm * nq, *c = T2 + nm * nq, *s1 = c + Q,
+           *s2 = s1 + n1;
+    const long e = blockIdx.x;
+    const double *g = geom + (deformed ? e * imf::geo_stride(7l * Q, sizeof(double)) : e * 7);
+    for (int i = threadIdx.x; i < nm * nq; i += blockDim.x) {
+        const double b = t.B[i], d = t.dB[i];
+        T0[i] = b * b;
+        T1[i] = d * d;
+        T2[i] = b * d;
+    }
+    double acc[2] = {0.0, 0.0};  // modes threadIdx.x + 256 u (at most 8^3 of them)
+    // tables per direction and factor of each term (w J, 00, 01, 02, 11, 12, 22)
+    for (int a = 0; a < 7; ++a) {
+        const double *X = a == 0 || a >= 4 ? T0 : a == 1 ? T1 : T2;
+        const double *Y = a == 4 ? T1 : a == 2 || a == 5 ? T2 : T0;
+        const double *Z = a == 6 ? T1 : a == 3 || a == 5 ? T2 : T0;
+        const double f = a == 0 ? lambda : a == 2 || a == 3 || a == 5 ? 2.0 : 1.0;
+        for (int i = threadIdx.x; i < Q; i += blockDim.x)
+            c[i] = f * (deformed ? g[(long)a * Q + i]
+                                 : g[a] * (t.w[i % nq] * t.w[i / nq % nq] * t.w[i / (nq * nq)]));
+        __syncthreads();
+        for (int o = threadIdx.x; o < n1; o += blockDim.x) {  // (k, j, p)
+            const double *row = c + o / nm * nq, *x = X + o % nm * nq;
+            double v = 0.0;
+            for (int i = 0; i < nq; ++i) v = fma(x[i], row[i], v);
+            s1[o] = v;
+        }
+        __syncthreads();
+        for (int o = threadIdx.x; o < n2; o += blockDim.x) {  // (k, q, p)
+            const int p = o % nm, q = o / nm % nm, k = o / (nm * nm);
+            double v = 0.0;
+            for (int j = 0; j < nq; ++j) v = fma(Y[q * nq + j], s1[(k * nq + j) * nm + p], v);
+            s2[o] = v;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {  // (r, q, p)
+            const int o = threadIdx.x + 256 * u;
+            if (o >= M) continue;
+            const double *z = Z + o / (nm * nm) * nq;
+            for (int k = 0; k < nq; ++k) acc[u] = fma(z[k], s2[k * nm * nm + o % (nm * nm)], acc[u]);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int o = threadIdx.x + 256 * u;
+        if (o < M) diag[e * M + o] = acc[u];
+    }
 }
 
 // The quad analogue (deformed [e][4Q]: Jw, Jw G00, Jw G01, Jw G11; regular [e][4]).
@@ -475,6 +510,14 @@ __global__ void inv_masked(long n, const unsigned char *__restrict__ mask, doubl
     if (i < n) d[i] = (mask && mask[i]) ? 0.0 : 1.0 / d[i];
 }
 
+// Scalars of the conjugate-gradient iteration, kept on the device so that the next kernels
+// can be queued without waiting for them.
+struct CgState {
+    double rho, mu, eps, alpha, beta, thr, rhs_mag;
+    int it;    // iterations as the reference counts them
+    int done;  // the tolerance is reached: the kernels of later iterations return at once
+};
+
 // r = mask0(b), x = 0
 __global__ void cg_init(long n, const unsigned char *__restrict__ mask, const double *__restrict__ b,
                         double *__restrict__ r, double *__restrict__ x)
@@ -494,20 +537,24 @@ __global__ void cg_precon(long n, const double *__restrict__ dinv, const double 
 }
 
 // p = w + beta p; q = s + beta q; x += alpha p; r -= alpha q; w = dinv r
-// (NekLinSysIterCG.cpp:186-204, with the Jacobi preconditioner fused)
-__global__ void cg_update(long n, double alpha, double beta, const double *__restrict__ dinv,
+// (NekLinSysIterCG.cpp:186-204, with the Jacobi preconditioner fused); the old w is dinv r
+// of the old r, both read here anyway
+__global__ void cg_update(long n, const CgState *__restrict__ st, const double *__restrict__ dinv,
                           double *__restrict__ p, double *__restrict__ q, double *__restrict__ w,
                           const double *__restrict__ s, double *__restrict__ x, double *__restrict__ r)
 {
+    if (st->done) return;
+    const double alpha = st->alpha, beta = st->beta;
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const double pi = w[i] + beta * p[i], qi = s[i] + beta * q[i];
+    const double di = dinv[i], r0 = r[i];
+    const double pi = di * r0 + beta * p[i], qi = s[i] + beta * q[i];
     p[i] = pi;
     q[i] = qi;
     x[i] += alpha * pi;
-    const double ri = r[i] - alpha * qi;
+    const double ri = r0 - alpha * qi;
     r[i] = ri;
-    w[i] = dinv[i] * ri;
+    w[i] = di * ri;
 }
 
 constexpr int RB = 256;
@@ -547,18 +594,19 @@ __global__ void dot3_partial(long n, const double *__restrict__ a, const double 
 // (r,w), (s,w), (r,r) for the conjugate-gradient step (grid-stride over the global modes,
 // part laid out as in dot3_partial, gridDim.x blocks: a fixed order, so reproducible).
 __global__ void assemble_dot3_kernel(long ng, const int *__restrict__ off,
-                                     const int *__restrict__ inv,
-                                     const signed char *__restrict__ sg,
+                                     const unsigned *__restrict__ inv,
                                      const double *__restrict__ loc,
                                      const unsigned char *__restrict__ mask,
                                      const double *__restrict__ extra,
+                                     const CgState *__restrict__ st,
                                      const double *__restrict__ r, const double *__restrict__ w,
                                      double *__restrict__ s_out, double *__restrict__ part)
 {
     __shared__ double sh[3][RB / 64];
+    if (st->done) return;
     double s0 = 0, s1 = 0, s2 = 0;
     for (long g = (long)blockIdx.x * RB + threadIdx.x; g < ng; g += (long)gridDim.x * RB) {
-        double sv = assemble_one(g, off, inv, sg, loc, mask);
+        double sv = assemble_one<false>(g, off, inv, loc, mask);
         // the Robin trace term of the global mode, when there is one (zero on Dirichlet modes)
         if (extra && !(mask && mask[g])) sv += extra[g];
         s_out[g] = sv;
@@ -586,22 +634,67 @@ __global__ void assemble_dot3_kernel(long ng, const int *__restrict__ off,
     }
 }
 
-__global__ void dot3_final(int nb, const double *__restrict__ part, double *__restrict__ out)
+// The three dot products of the block partial sums and the iteration's scalars from them
+// (NekLinSysIterCG.cpp:160-204).  One workgroup, every partial loaded at once: with 256 threads
+// walking the sums one after the other it took 14.7 us of an iteration's 113 (8 000 elements of
+// 6 modes), now 4.  WHAT: 0 the right-hand side's magnitude, 1 the first residual, 2 the first
+// direction, 3 an iteration.
+constexpr int FB = 1024;
+template <int WHAT>
+__global__ __launch_bounds__(FB) void cg_scalars(int nb, const double *__restrict__ part, double tol,
+                                                 CgState *__restrict__ st)
 {
-    __shared__ double sh[RB / 64];
-    for (int c = 0; c < 3; ++c) {
-        double s = 0;
-        for (int i = threadIdx.x; i < nb; i += RB) s += part[(long)c * nb + i];
+    __shared__ double sh[3][FB / 64];
+    if (WHAT >= 2 && st->done) return;
+    double v[3] = {0.0, 0.0, 0.0};
+    for (int i0 = 0; i0 < nb; i0 += 4 * FB) {
+        double x[3][4];
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-        if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double t = 0;
-            for (int w = 0; w < RB / 64; ++w) t += sh[w];
-            out[c] = t;
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int i = i0 + u * FB + (int)threadIdx.x;
+                x[c][u] = i < nb ? part[(long)c * nb + i] : 0.0;
+            }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) v[c] += (x[c][0] + x[c][1]) + (x[c][2] + x[c][3]);
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) v[c] += __shfl_xor(v[c], off);
+        if ((threadIdx.x & 63) == 0) sh[c][threadIdx.x >> 6] = v[c];
+    }
+    __syncthreads();
+    if (threadIdx.x) return;
+    double h[3];
+    for (int c = 0; c < 3; ++c) {
+        h[c] = 0.0;
+        for (int w = 0; w < FB / 64; ++w) h[c] += sh[c][w];
+    }
+    if constexpr (WHAT == 0) {
+        st->rhs_mag = h[0] > 1e-6 ? h[0] : 1.0;
+        st->thr = tol * tol * st->rhs_mag;
+    } else if constexpr (WHAT == 1) {
+        st->eps = h[2];
+        st->it = 0;
+        st->done = !(h[2] >= st->thr);
+    } else if constexpr (WHAT == 2) {
+        st->rho = h[0];
+        st->alpha = h[0] / h[1];
+        st->beta = 0.0;
+        st->it = 1;
+    } else {
+        st->eps = h[2];
+        ++st->it;
+        if (h[2] < st->thr) {
+            st->done = 1;
+            return;
         }
-        __syncthreads();
+        const double beta = h[0] / st->rho;
+        st->alpha = h[0] / (h[1] - h[0] * beta / st->alpha);
+        st->beta = beta;
+        st->rho = h[0];
     }
 }
 
@@ -629,7 +722,8 @@ __global__ void csr_diag_add(long ng, const int *__restrict__ off, const int *__
         if (col[k] == g) d[g] += val[k];
 }
 
-// blocks of the fused assembly + dot pass (16 per CU on a 256-CU device)
+// blocks of the fused assembly + dot pass (16 per CU on a 256-CU device; cg_scalars loads
+// their partial sums in one go)
 constexpr long kAsmParts = 4096;
 
 }  // namespace
@@ -642,14 +736,17 @@ struct imf_asm_s {
     std::vector<long> loff;  // first local coefficient of each element (nElmt + 1)
     int *d_l2g = nullptr;
     signed char *d_sg = nullptr;
-    int *d_off = nullptr, *d_inv = nullptr;  // inverse map (CSR), 32-bit
+    int *d_off = nullptr;      // inverse map (CSR), 32-bit, signs in the top bits
+    unsigned *d_inv = nullptr;
     unsigned char *d_mask = nullptr;  // global Dirichlet mask (NULL without Dirichlet)
     // Robin trace terms: a sparse matrix over the global modes (CSR), and R w of the solve
     long r_nnz = 0;
     int *d_roff = nullptr, *d_rcol = nullptr;
     double *d_rval = nullptr, *d_rw = nullptr;
     // solver workspace (allocated on the first solve)
-    double *d_ws = nullptr, *d_loc = nullptr, *d_part = nullptr, *d_dots = nullptr;
+    double *d_ws = nullptr, *d_loc = nullptr, *d_part = nullptr;
+    CgState *d_state = nullptr, *h_state = nullptr;  // device; two pinned copies
+    hipEvent_t ev[2] = {nullptr, nullptr};
     int nparts = 0;
     // operators, their geometry versions and lambdas the cached diagonal belongs to
     std::vector<std::tuple<const void *, unsigned long, double>> diag_key;
@@ -664,11 +761,12 @@ namespace {
     } while (0)
 
 // out = mask0(Assemble(H(GlobalToLocal(w))))  (GlobalLinSysIterativeFull::v_DoMatrixMultiply)
-// with the partial sums of (r,w), (out,w), (r,r) taken in the assembly pass.  ops[g] acts on
+// with the partial sums of (r,w), (out,w), (r,r) taken in the assembly pass and the
+// iteration's scalars from them (first: those of the first direction).  ops[g] acts on
 // the next ops[g]->nElmt elements (one operator per order, as the reference keeps one
 // collection per expansion type).
 int apply_global_dots(imf_asm a, int nops, const imf_op *ops, const double *w, const double *r,
-                      double *out, hipStream_t s)
+                      double *out, bool first, hipStream_t s)
 {
     double *l0 = a->d_loc, *l1 = a->d_loc + a->nloc;
     const bool any_aniso = std::any_of(ops, ops + nops, [](const imf_op o) { return o->aniso; });
@@ -676,7 +774,8 @@ int apply_global_dots(imf_asm a, int nops, const imf_op *ops, const double *w, c
         long e0 = 0;
         for (int g = 0; g < nops; ++g) {
             const long o = a->loff[e0];
-            if (int st = imf_apply_gather_device(ops[g], w, a->d_l2g + o, a->d_sg + o, l1 + o, s))
+            if (int st = imf_apply_gather_device(ops[g], w, a->d_l2g + o, a->d_sg + o, l1 + o,
+                                                 &a->d_state->done, s))
                 return st;
             e0 += ops[g]->nElmt;
         }
@@ -692,9 +791,11 @@ int apply_global_dots(imf_asm a, int nops, const imf_op *ops, const double *w, c
     if (a->r_nnz)
         csr_spmv<<<nblk(a->ng), RB, 0, s>>>(a->ng, a->d_roff, a->d_rcol, a->d_rval, w, a->d_rw);
     const int nb = (int)std::min<long>(kAsmParts, nblk(a->ng));
-    assemble_dot3_kernel<<<nb, RB, 0, s>>>(a->ng, a->d_off, a->d_inv, a->d_sg, l1, a->d_mask,
-                                           a->r_nnz ? a->d_rw : nullptr, r, w, out, a->d_part);
-    dot3_final<<<1, RB, 0, s>>>(nb, a->d_part, a->d_dots);
+    assemble_dot3_kernel<<<nb, RB, 0, s>>>(a->ng, a->d_off, a->d_inv, l1, a->d_mask,
+                                           a->r_nnz ? a->d_rw : nullptr, a->d_state, r, w, out,
+                                           a->d_part);
+    if (first) cg_scalars<2><<<1, FB, 0, s>>>(nb, a->d_part, 0.0, a->d_state);
+    else cg_scalars<3><<<1, FB, 0, s>>>(nb, a->d_part, 0.0, a->d_state);
     ACHECK(hipGetLastError(), "assembly kernels");
     return IMF_OK;
 }
@@ -764,11 +865,11 @@ static int create_any(int shape, int nElmt, const int *nm, const long long *vert
     std::vector<int> off(ng + 1, 0);
     for (long i = 0; i < a->nloc; ++i)
         if (sg[i]) ++off[m[i] + 1], ++nused;
-    std::vector<int> inv(std::max<long>(nused, 1));
+    std::vector<unsigned> inv(std::max<long>(nused, 1));
     for (long g = 0; g < ng; ++g) off[g + 1] += off[g];
     std::vector<int> fill(off.begin(), off.end() - 1);
     for (long i = 0; i < a->nloc; ++i)
-        if (sg[i]) inv[fill[m[i]]++] = (int)i;
+        if (sg[i]) inv[fill[m[i]]++] = (unsigned)i | (sg[i] < 0 ? 0x80000000u : 0u);
     std::vector<unsigned char> gmask;
     if (a->dirichlet) {
         gmask.assign(ng, 0);
@@ -783,13 +884,13 @@ static int create_any(int shape, int nElmt, const int *nm, const long long *vert
     if ((e = hipMalloc(&a->d_l2g, a->nloc * sizeof(int))) != hipSuccess ||
         (e = hipMalloc(&a->d_sg, a->nloc)) != hipSuccess ||
         (e = hipMalloc(&a->d_off, (ng + 1) * sizeof(int))) != hipSuccess ||
-        (e = hipMalloc(&a->d_inv, inv.size() * sizeof(int))) != hipSuccess ||
+        (e = hipMalloc(&a->d_inv, inv.size() * sizeof(unsigned))) != hipSuccess ||
         (a->dirichlet && (e = hipMalloc(&a->d_mask, ng)) != hipSuccess))
         return cleanup(afail(IMF_ERR_HIP, std::string("hipMalloc(assembly): ") + hipGetErrorString(e)));
     if ((e = hipMemcpy(a->d_l2g, m.data(), a->nloc * sizeof(int), hipMemcpyHostToDevice)) != hipSuccess ||
         (e = hipMemcpy(a->d_sg, sg.data(), a->nloc, hipMemcpyHostToDevice)) != hipSuccess ||
         (e = hipMemcpy(a->d_off, off.data(), (ng + 1) * sizeof(int), hipMemcpyHostToDevice)) != hipSuccess ||
-        (e = hipMemcpy(a->d_inv, inv.data(), inv.size() * sizeof(int), hipMemcpyHostToDevice)) != hipSuccess ||
+        (e = hipMemcpy(a->d_inv, inv.data(), inv.size() * sizeof(unsigned), hipMemcpyHostToDevice)) != hipSuccess ||
         (a->dirichlet && (e = hipMemcpy(a->d_mask, gmask.data(), ng, hipMemcpyHostToDevice)) != hipSuccess))
         return cleanup(afail(IMF_ERR_HIP, std::string("hipMemcpy(assembly): ") + hipGetErrorString(e)));
     *out = a;
@@ -869,9 +970,12 @@ int imf_assembly_destroy(imf_asm a)
     if (!a) return IMF_OK;
     for (void *p : {(void *)a->d_l2g, (void *)a->d_sg, (void *)a->d_off, (void *)a->d_inv,
                     (void *)a->d_mask, (void *)a->d_ws, (void *)a->d_loc, (void *)a->d_part,
-                    (void *)a->d_dots, (void *)a->d_roff, (void *)a->d_rcol, (void *)a->d_rval,
+                    (void *)a->d_state, (void *)a->d_roff, (void *)a->d_rcol, (void *)a->d_rval,
                     (void *)a->d_rw})
         if (p) (void)hipFree(p);
+    if (a->h_state) (void)hipHostFree(a->h_state);
+    for (hipEvent_t ev : a->ev)
+        if (ev) (void)hipEventDestroy(ev);
     delete a;
     return IMF_OK;
 }
@@ -943,8 +1047,8 @@ int imf_global_to_local_device(imf_asm a, const double *d_global, double *d_loca
 int imf_assemble_device(imf_asm a, const double *d_local, double *d_global, void *stream)
 {
     if (!a || !d_global || !d_local) return afail(IMF_ERR_ARG, "imf_assemble_device: null argument");
-    assemble_kernel<<<nblk(a->ng), RB, 0, (hipStream_t)stream>>>(a->ng, a->d_off, a->d_inv, a->d_sg,
-                                                                d_local, nullptr, d_global);
+    assemble_kernel<false><<<nblk(a->ng), RB, 0, (hipStream_t)stream>>>(a->ng, a->d_off, a->d_inv,
+                                                                       d_local, nullptr, d_global);
     ACHECK(hipGetLastError(), "assemble_kernel");
     return IMF_OK;
 }
@@ -983,14 +1087,18 @@ int imf_helmsolve_cg_groups_device(imf_asm a, int nops, const imf_op *ops, const
                                   "assembly's elements");
     hipStream_t s = (hipStream_t)stream;
     const long ng = a->ng;
-    if (!a->d_ws) {
+    if (!a->ev[1]) {  // the last piece of the workspace; after a failure, what is missing
         a->nparts = (int)std::min<long>(1024, (ng + RB - 1) / RB);
-        ACHECK(hipMalloc(&a->d_ws, 6 * ng * sizeof(double)), "hipMalloc(cg)");
-        ACHECK(hipMalloc(&a->d_loc, 2 * a->nloc * sizeof(double)), "hipMalloc(cg)");
         // block partial sums: dot3_partial's or the fused assembly pass's blocks
         const long np = std::max<long>(a->nparts, std::min<long>(kAsmParts, nblk(ng)));
-        ACHECK(hipMalloc(&a->d_part, 3 * np * sizeof(double)), "hipMalloc(cg)");
-        ACHECK(hipMalloc(&a->d_dots, 4 * sizeof(double)), "hipMalloc(cg)");
+        if (!a->d_ws) ACHECK(hipMalloc(&a->d_ws, 6 * ng * sizeof(double)), "hipMalloc(cg)");
+        if (!a->d_loc) ACHECK(hipMalloc(&a->d_loc, 2 * a->nloc * sizeof(double)), "hipMalloc(cg)");
+        if (!a->d_part) ACHECK(hipMalloc(&a->d_part, 3 * np * sizeof(double)), "hipMalloc(cg)");
+        if (!a->d_state) ACHECK(hipMalloc(&a->d_state, sizeof(CgState)), "hipMalloc(cg)");
+        if (!a->h_state)
+            ACHECK(hipHostMalloc(&a->h_state, 2 * sizeof(CgState), hipHostMallocDefault), "hipHostMalloc(cg)");
+        for (hipEvent_t &ev : a->ev)
+            if (!ev) ACHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate(cg)");
         a->diag_key.clear();
     }
     double *r = a->d_ws, *p = r + ng, *q = p + ng, *w = q + ng, *sv = w + ng, *dinv = sv + ng;
@@ -1014,73 +1122,64 @@ int imf_helmsolve_cg_groups_device(imf_asm a, int nops, const imf_op *ops, const
                 ACHECK(imf::launch_aniso_diag(aniso_args(op, nullptr, nullptr, 1, 0, 0), dl, s),
                        "anisotropic diagonal");
             else if (a->shape == imf::kHex)
-                helm_diag_hex<<<nblk(n), RB, 0, s>>>(t, nm, nq, op->nElmt, op->deformed, op->lambda,
-                                                    (const double *)op->d_geom, dl);
+                helm_diag_hex<<<op->nElmt, 256,
+                                sizeof(double) * (3 * nm * nq + nq * nq * nq + nq * nq * nm + nq * nm * nm),
+                                s>>>(t, nm, nq, op->deformed, op->lambda,
+                                     (const double *)op->d_geom, dl);
             else
                 helm_diag_quad<<<nblk(n), RB, 0, s>>>(t, nm, nq, op->nElmt, op->deformed, op->lambda,
                                                      (const double *)op->d_geom, dl);
             e0 += op->nElmt;
         }
-        assemble_kernel<<<nblk(ng), RB, 0, s>>>(ng, a->d_off, a->d_inv, nullptr, a->d_loc, nullptr, dinv);
+        assemble_kernel<true><<<nblk(ng), RB, 0, s>>>(ng, a->d_off, a->d_inv, a->d_loc, nullptr, dinv);
         if (a->r_nnz)
             csr_diag_add<<<nblk(ng), RB, 0, s>>>(ng, a->d_roff, a->d_rcol, a->d_rval, dinv);
         inv_masked<<<nblk(ng), RB, 0, s>>>(ng, a->d_mask, dinv);
         ACHECK(hipGetLastError(), "diagonal kernels");
         a->diag_key = key;
     }
-    double h[4];
-    auto read_dots = [&]() -> int {
-        ACHECK(hipMemcpyAsync(h, a->d_dots, 3 * sizeof(double), hipMemcpyDeviceToHost, s), "copy");
-        ACHECK(hipStreamSynchronize(s), "sync");
-        return IMF_OK;
-    };
-    auto dots = [&](const double *x0, const double *x1, const double *x2) -> int {
+    auto dots = [&](const double *x0, const double *x1, const double *x2) {
         dot3_partial<<<a->nparts, RB, 0, s>>>(ng, x0, x1, x2, a->d_part);
-        dot3_final<<<1, RB, 0, s>>>(a->nparts, a->d_part, a->d_dots);
-        ACHECK(hipGetLastError(), "dot kernels");
-        return read_dots();
     };
-    // s = A w with (r,w), (s,w), (r,r) in the same pass
-    auto apply_dots = [&]() -> int {
-        if (int st = apply_global_dots(a, nops, ops, w, r, sv, s)) return st;
-        return read_dots();
-    };
-    // rhs magnitude over all global modes (Set_Rhs_Magnitude)
-    if (int st = dots(d_rhs, d_rhs, d_rhs)) return st;
-    const double rhs_mag = h[0] > 1e-6 ? h[0] : 1.0;
+    // rhs magnitude over all global modes (Set_Rhs_Magnitude), the first residual and the first
+    // direction; then iterations in groups of four, a copy of the scalars after each.  The host
+    // waits for the scalars of the group before the one it has just queued, so the device always
+    // has work; iterations queued past the last one return at once.
+    dots(d_rhs, d_rhs, d_rhs);
+    cg_scalars<0><<<1, FB, 0, s>>>(a->nparts, a->d_part, tol, a->d_state);
     cg_init<<<nblk(ng), RB, 0, s>>>(ng, a->d_mask, d_rhs, r, d_x);
-    ACHECK(hipGetLastError(), "cg_init");
-    if (int st = dots(r, r, r)) return st;
-    double eps = h[2];
-    const double thr = tol * tol * rhs_mag;
-    int it = 0;
-    if (eps >= thr) {
-        cg_precon<<<nblk(ng), RB, 0, s>>>(ng, dinv, r, w);
-        if (int st = apply_dots()) return st;  // (r,w), (s,w), (r,r)
-        double rho = h[0], mu = h[1];
-        double beta = 0.0, alpha = rho / mu;
-        it = 1;
-        zero_kernel<<<nblk(2 * ng), RB, 0, s>>>(2 * ng, p);  // p and q
-        for (;;) {
-            if (it > max_iter) {
-                if (iterations) *iterations = it;
-                if (residual) *residual = std::sqrt(eps / rhs_mag);
-                return afail(IMF_ERR_STATE, "Exceeded maximum number of iterations");
-            }
-            cg_update<<<nblk(ng), RB, 0, s>>>(ng, alpha, beta, dinv, p, q, w, sv, d_x, r);
-            if (int st = apply_dots()) return st;
-            const double rho_new = h[0];
-            mu = h[1];
-            eps = h[2];
-            ++it;
-            if (eps < thr) break;
-            beta = rho_new / rho;
-            alpha = rho_new / (mu - rho_new * beta / alpha);
-            rho = rho_new;
+    dots(r, r, r);
+    cg_scalars<1><<<1, FB, 0, s>>>(a->nparts, a->d_part, tol, a->d_state);
+    cg_precon<<<nblk(ng), RB, 0, s>>>(ng, dinv, r, w);
+    zero_kernel<<<nblk(2 * ng), RB, 0, s>>>(2 * ng, p);  // p and q
+    ACHECK(hipGetLastError(), "cg set-up kernels");
+    if (int st = apply_global_dots(a, nops, ops, w, r, sv, true, s)) return st;
+    constexpr int kGroup = 4;
+    CgState last{};
+    long queued = 0;
+    for (int b = 0, first = 1;; b ^= 1, first = 0) {
+        const long upto = std::min<long>(std::max(max_iter, 0), queued + kGroup);
+        for (; queued < upto; ++queued) {
+            cg_update<<<nblk(ng), RB, 0, s>>>(ng, a->d_state, dinv, p, q, w, sv, d_x, r);
+            if (int st = apply_global_dots(a, nops, ops, w, r, sv, false, s)) return st;
+        }
+        ACHECK(hipMemcpyAsync(a->h_state + b, a->d_state, sizeof(CgState), hipMemcpyDeviceToHost, s), "copy");
+        ACHECK(hipEventRecord(a->ev[b], s), "event");
+        if (!first) {
+            ACHECK(hipEventSynchronize(a->ev[b ^ 1]), "sync");
+            last = a->h_state[b ^ 1];
+            if (last.done) break;
+        }
+        if (queued >= max_iter) {
+            ACHECK(hipEventSynchronize(a->ev[b]), "sync");
+            last = a->h_state[b];
+            break;
         }
     }
-    if (iterations) *iterations = it;
-    if (residual) *residual = std::sqrt(eps / rhs_mag);
+    ACHECK(hipStreamSynchronize(s), "sync");
+    if (iterations) *iterations = last.it;
+    if (residual) *residual = std::sqrt(last.eps / last.rhs_mag);
+    if (!last.done) return afail(IMF_ERR_STATE, "Exceeded maximum number of iterations");
     return IMF_OK;
 }
 

@@ -383,7 +383,8 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_mass_kernel(
 // components (Jw, JwG00, JwG01, JwG02, JwG11, JwG12, JwG22) at c*Q; regular [e][7]
 // (J, J G00, ...), weights applied in the kernel.
 // GATHER: `in` is a global vector read through (gmap, gsign), as GlobalToLocal would
-// expand it, so the solver's operator needs no local copy of its input.
+// expand it, so the solver's operator needs no local copy of its input; skip (may be null)
+// points to a device flag that makes the kernel return (an iteration queued past the last).
 // MANY: nvec vectors per launch (vector v at in + v*ldin, out + v*ldout), the operator
 // applied to each in turn by the same workgroup; deformed geometry is staged in LDS once
 // (when the element's 7Q values fit beside the work buffers) and read from there for
@@ -413,8 +414,9 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_helmholtz_kernel(
     const Tab<NM, NQ, T> tab, int nElmt, T lambda, const T *__restrict__ in,
     const T *__restrict__ geom, T *__restrict__ out, const int *__restrict__ gmap = nullptr,
     const signed char *__restrict__ gsign = nullptr, int nvec = 1, long ldin = 0,
-    long ldout = 0)
+    long ldout = 0, const int *__restrict__ skip = nullptr)
 {
+    if (GATHER && skip && *skip) return;
     using C = HexCfg<NQ>;
     using Lb = HexLds<NM, NQ>;
     constexpr int M = Lb::M, Q = Lb::Q, TPE = C::TPE;

@@ -29,7 +29,7 @@ hipError_t launch_hex(const LaunchArgs &a)
         if constexpr (std::is_same_v<T, double>) {
             if (a.gmap) {
                 hex_helmholtz_kernel<NM, NQ, T, GEO, true><<<grid, block, 0, a.stream>>>(
-                    tab, a.nElmt, T(a.lambda), in, geom, out, a.gmap, a.gsign);
+                    tab, a.nElmt, T(a.lambda), in, geom, out, a.gmap, a.gsign, 1, 0, 0, a.skip);
                 return hipGetLastError();
             }
         }

@@ -64,6 +64,8 @@ imf::AnisoArgs aniso_args(const imf_op_s *op, const void *in, void *out, int nve
 
 // FP64 hex Helmholtz with its input gathered from a global vector: out = H(local), where
 // local[i] = gsign[i] * glob[gmap[i]] (GlobalToLocal fused into the kernel's load).
-// Library-internal (used by the assembled solver); defined in mf_capi.hip.
+// skip (device, may be null): nothing is done when it holds a non-zero value at the time the
+// kernel runs.  Library-internal (used by the assembled solver); defined in mf_capi.hip.
 int imf_apply_gather_device(imf_op_s *op, const double *glob, const int *gmap,
-                            const signed char *gsign, double *out, hipStream_t stream);
+                            const signed char *gsign, double *out, const int *skip,
+                            hipStream_t stream);

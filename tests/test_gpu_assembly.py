@@ -439,3 +439,26 @@ def test_preconditioner_follows_a_recreated_operator():
         print(f"scale {s}: iterations {it1} / {it2}")
         assert it1 == it2
         assert torch.equal(x1, x2)
+
+
+@pytest.mark.parametrize("nm,nq,lam", [(2, 4, 1.0), (4, 5, 10.0), (8, 9, 10.0), (7, 14, 2.0)])
+def test_iteration_limit_at_and_around_convergence(nm, nq, lam):
+    """Iterations are queued in groups ahead of the convergence test: the solve stops at the same
+    iteration with any limit that allows it (x bit for bit the same), one short of it reports
+    limit + 1 iterations as the reference does, and a zero right-hand side takes none."""
+    verts, ids = _mesh(2, True, seed=4, jitter=0.05)
+    print(f"[case] cg limits nm={nm} nq={nq}", flush=True)
+    A, Hop, rhs, _ = _gpu_problem(verts, ids, nm, nq, lam)
+    x, it, res = A.helmsolve(Hop, rhs, tol=1e-10)
+    assert res <= 1e-10 and it >= 2
+    for limit in (it - 1, it, it + 3, it + 9):
+        y, jt, rs = A.helmsolve(Hop, rhs, tol=1e-10, max_iter=limit)
+        assert jt == it and rs == res and torch.equal(x, y)
+    for limit in {0, max(it - 2, 0)}:
+        with pytest.raises(H.MFError, match="maximum number of iterations"):
+            A.helmsolve(Hop, rhs, tol=1e-10, max_iter=limit)
+    z, kt, _ = A.helmsolve(Hop, torch.zeros_like(rhs), tol=1e-10)
+    assert kt == 0 and not z.any()
+    # the preconditioner's diagonal: with it the solve takes no more iterations than the bound of
+    # a Jacobi-scaled system of this size (a wrong diagonal takes several times more)
+    assert it < 60 * nm
