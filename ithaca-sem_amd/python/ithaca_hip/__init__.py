@@ -82,9 +82,12 @@ def _np_ptr(a):
 
 
 def _stream_ptr(stream):
-    if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    """The hipStream_t of a torch stream, or of the current device's current stream.  The raw
+    handle of the current stream is asked for directly: torch.cuda.current_stream() builds a
+    Stream object, 2.6 us of a call whose launch takes 4."""
+    if stream is not None:
+        return stream.cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def basis_modified_a(nm, nq):
@@ -350,9 +353,10 @@ class Operator:
         assert inp.numel() == self.in_size
         if out is None:
             out = torch.empty(self.out_size, dtype=self.dtype, device=inp.device)
-        assert out.is_cuda and out.dtype == self.dtype and out.numel() == self.out_size
-        _check(lib().imf_apply_device(self._h, ctypes.c_void_p(inp.data_ptr()),
-                                      ctypes.c_void_p(out.data_ptr()), _stream_ptr(stream)))
+        else:
+            assert out.is_cuda and out.dtype == self.dtype and out.numel() == self.out_size
+        _check(lib().imf_apply_device(self._h, inp.data_ptr(), out.data_ptr(),
+                                      _stream_ptr(stream)))
         return out
 
     def apply_transpose(self, inp, out=None, stream=None):
@@ -362,8 +366,7 @@ class Operator:
         if out is None:
             out = torch.empty(self.in_size, dtype=self.dtype, device=inp.device)
         assert out.numel() == self.in_size
-        _check(lib().imf_apply_transpose_device(self._h, ctypes.c_void_p(inp.data_ptr()),
-                                                ctypes.c_void_p(out.data_ptr()),
+        _check(lib().imf_apply_transpose_device(self._h, inp.data_ptr(), out.data_ptr(),
                                                 _stream_ptr(stream)))
         return out
 
@@ -377,9 +380,8 @@ class Operator:
                               device=inp.device)
         assert out.is_cuda and out.dtype == self.dtype and out.dim() == 2 and out.stride(1) == 1
         assert out.shape[0] == inp.shape[0] and out.shape[1] >= self.out_size
-        _check(lib().imf_apply_many_device(self._h, inp.shape[0], ctypes.c_void_p(inp.data_ptr()),
-                                           inp.stride(0), ctypes.c_void_p(out.data_ptr()),
-                                           out.stride(0), _stream_ptr(stream)))
+        _check(lib().imf_apply_many_device(self._h, inp.shape[0], inp.data_ptr(), inp.stride(0),
+                                           out.data_ptr(), out.stride(0), _stream_ptr(stream)))
         return out
 
     def apply_host(self, inp):

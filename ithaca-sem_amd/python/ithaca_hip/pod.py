@@ -17,7 +17,7 @@ import ctypes
 import numpy as np
 import torch
 
-from . import FP64, MFError, Operator
+from . import FP64, MFError, Operator, _stream_ptr
 from . import rom as _rom
 
 GRAM_FP64, GRAM_FP32X3, GRAM_BF16X3 = 0, 1, 2
@@ -43,7 +43,7 @@ def _lib():
 
 
 def _s(stream=None):
-    return ctypes.c_void_p((stream or torch.cuda.current_stream()).cuda_stream)
+    return ctypes.c_void_p(_stream_ptr(stream))
 
 
 def gram(X, Y=None, mode=GRAM_FP64, out=None, accumulate=False, work=None, stream=None,

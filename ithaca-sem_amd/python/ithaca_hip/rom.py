@@ -9,7 +9,7 @@ import ctypes
 import numpy as np
 import torch
 
-from . import LIB_PATH, MFError
+from . import LIB_PATH, MFError, _stream_ptr
 
 LU_FP64, LU_FP32_IR, LU_FP32_IR_FALLBACK = 0, 1, 2
 KINDS = ("normalised", "literal", "nonsymmetric")
@@ -51,7 +51,7 @@ def _ptr(t):
 
 
 def _stream(s):
-    return ctypes.c_void_p((s or torch.cuda.current_stream()).cuda_stream)
+    return ctypes.c_void_p(_stream_ptr(s))
 
 
 class Batch:
