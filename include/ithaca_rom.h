@@ -63,7 +63,8 @@ int irom_batch_solve(irom_batch b, int method, int transpose, const double *d_A,
                      int max_iter, int *d_iters, int *d_status, void *stream);
 
 /* Tile variant used by irom_batch_solve for a method: set explicitly, or choose by timing
- * every variant on the given data (the autotuner; returns the chosen index).  */
+ * every variant on the given data (the autotuner; returns the chosen index).  The variants
+ * are shapes of the mixed-precision kernel; the FP64 kernel has one, whatever is set. */
 int irom_batch_num_variants(void);
 const char *irom_batch_variant_name(int v);
 int irom_batch_set_variant(irom_batch b, int method, int v);

@@ -263,3 +263,60 @@ def test_status_codes_and_degenerate_batches(method):
     x1 = B1.solve(_dev(one["A"]), _dev(one["theta"]), _dev(one["b"]), method=method)
     r1 = R.solve(one)
     assert np.linalg.norm(x1.cpu().numpy() - r1) <= TOL * np.linalg.norm(r1)
+
+
+@pytest.mark.parametrize("transpose", [False, True])
+def test_fp64_solves_at_panel_edges(transpose):
+    """Sizes around the panels of 16 columns and the 64 / 128 / 192 row limits of the FP64 kernel's
+    paths, one to nine terms, matrices that need row interchanges (Gaussian; a permuted diagonal;
+    rows scaled over 12 decades), two singular ones.  Bar: the normwise backward error of partial
+    pivoting, here at most 4 N eps with its growth factors below 8, for every instance."""
+    N = [1, 2, 3, 15, 16, 17, 31, 32, 33, 48, 63, 64, 65, 80, 127, 128, 129, 143, 144, 145, 160, 191, 192,
+         193, 208, 240, 255, 256]
+    kinds = ["gauss", "perm", "scaled"]
+    rng = np.random.default_rng(11)
+    sizes, mats, qs = [], [], []
+    for n in N:
+        for kind in kinds:
+            Q = 1 + (n + len(kind)) % 9
+            M = rng.standard_normal((Q, n, n))
+            if kind == "perm":
+                M *= 1e-3
+                M[0] += np.diag(rng.uniform(1, 2, n))[rng.permutation(n)]
+            elif kind == "scaled":
+                M *= 10.0 ** rng.uniform(-6, 6, n)[None, :, None]
+            sizes.append(n)
+            qs.append(Q)
+            mats.append(M)
+    for n in (40, 200):  # a zero row and column: singular
+        M = rng.standard_normal((1, n, n))
+        M[0, n // 2] = 0.0
+        M[0, :, n // 2] = 0.0
+        sizes.append(n)
+        qs.append(1)
+        mats.append(M)
+    batch = rom.Batch(sizes, qs)
+    theta = rng.uniform(0.1, 1.0, batch.t_size)
+    b = rng.standard_normal(batch.v_size)
+    A = _dev(np.concatenate([m.ravel() for m in mats]))
+    status = torch.full((batch.n,), -1, dtype=torch.int32, device="cuda")
+    print("[case] fp64 panel edges", transpose, flush=True)
+    x = batch.solve(A, _dev(theta), _dev(b), transpose=transpose, status=status).cpu().numpy()
+    st = status.cpu().numpy()
+    lam = rng.standard_normal(batch.v_size)
+    grad = batch.param_grad(A, _dev(lam), _dev(x)).cpu().numpy()
+    for i, (n, Q, M) in enumerate(zip(sizes, qs, mats)):
+        if i >= len(sizes) - 2:
+            assert st[i] == 1
+            continue
+        th = theta[batch.t_off[i]:batch.t_off[i] + Q]
+        Am = np.tensordot(th, M, 1)
+        Am = Am.T if transpose else Am
+        sl = slice(batch.v_off[i], batch.v_off[i] + n)
+        r = b[sl] - Am @ x[sl]
+        back = np.abs(r).max() / (np.abs(Am).sum(1).max() * np.abs(x[sl]).max() + np.abs(b[sl]).max())
+        assert st[i] == 0 and back < 4 * max(n, 4) * 2.2e-16, (n, Q, back)
+        ref = np.array([-lam[sl] @ (M[q] @ x[sl]) for q in range(Q)])
+        scale = np.array([np.abs(lam[sl]) @ (np.abs(M[q]) @ np.abs(x[sl])) for q in range(Q)])
+        got = grad[batch.t_off[i]:batch.t_off[i] + Q]
+        assert np.abs(got - ref).max() < 1e-14 * n * scale.max()
