@@ -49,13 +49,37 @@ struct DTab {
 };
 
 // Launch shape of the hex kernels: NQ*NQ threads own the NQ*NQ point columns of one
-// element; small elements are packed several to a 64-lane wavefront.
-template <int NQ>
+// element; small elements are packed several to a 64-lane wavefront.  WIDE packs them into
+// 256 threads instead, which uses more of the lanes (6 points: 252 of 256 against 36 of 64)
+// at the price of barriers between the waves.
+template <int NQ, bool WIDE = false>
 struct HexCfg {
     static constexpr int TPE = NQ * NQ;
-    static constexpr int EPB = (64 / TPE) > 0 ? 64 / TPE : 1;
+    static constexpr int EPB = WIDE ? 256 / TPE : (64 / TPE) > 0 ? 64 / TPE : 1;
     static constexpr int BLOCK = ((EPB * TPE + 63) / 64) * 64;
 };
+
+// The table argument, read where the kernel's arguments lie; for kernels whose first argument
+// it is.  Each call is a new place to the compiler, so a table used through it is loaded where
+// it is used.  Otherwise the compiler loads every table into scalar registers at the start and
+// moves what does not fit to lanes of vector registers (8 modes, 9 points: 670 values, two
+// moves back for each product), or, with a lane-dependent index and some 300 uses, copies the
+// whole argument to scratch for every thread.  At 12e6 points, held / read again, in us:
+// Helmholtz regular 8,9 2 056/108 and 7,8 95/86, deformed 8,9 258/180 and 7,8 152/136;
+// BwdTrans 8,9 70/39; quad Helmholtz regular 8,10 1 345/88.  AGAIN = false leaves the table to
+// the compiler, for kernels that it slows down.
+template <bool AGAIN = true, typename TabT>
+__device__ __forceinline__ decltype(auto) reread(const TabT &tab)
+{
+    if constexpr (AGAIN) {
+        auto p = (const __attribute__((address_space(4))) TabT *)
+            __builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(p));
+        return (*p);
+    } else {
+        return (tab);
+    }
+}
 
 // Launch shape of the quad kernels: NQ threads own the NQ point lines of one element;
 // 256-thread blocks hold 4 * floor(64 / NQ) elements.

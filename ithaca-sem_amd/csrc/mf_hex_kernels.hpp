@@ -52,11 +52,11 @@ struct HexLds {
 // coefficients (nv*M scalars from src) into the padded pencil buffers buf(slot).
 // All of a thread's loads are issued before its first LDS store, so the span costs one
 // memory round trip rather than one per loop iteration.
-template <int NM, int NQ, typename T, typename BufFn>
+template <int NM, int NQ, typename C, typename T, typename BufFn>
 __device__ __forceinline__ void load_modes_block(const T *__restrict__ src, int nv, BufFn buf)
 {
     constexpr int M = NM * NM * NM;
-    constexpr int BLOCK = HexCfg<NQ>::BLOCK, PER = (HexCfg<NQ>::EPB * M + BLOCK - 1) / BLOCK;
+    constexpr int BLOCK = C::BLOCK, PER = (C::EPB * M + BLOCK - 1) / BLOCK;
     T v[PER];
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
@@ -77,14 +77,14 @@ __device__ __forceinline__ void load_modes_block(const T *__restrict__ src, int 
 // The same from a global vector: coefficient f of the block is gsign[f] * glob[gmap[f]]
 // (gmap, gsign offset to the block's first element; the map reads are coalesced, the
 // gather follows the global numbering).
-template <int NM, int NQ, typename T, typename BufFn>
+template <int NM, int NQ, typename C, typename T, typename BufFn>
 __device__ __forceinline__ void load_modes_block_gather(const T *__restrict__ glob,
                                                         const int *__restrict__ gmap,
                                                         const signed char *__restrict__ gsign,
                                                         int nv, BufFn buf)
 {
     constexpr int M = NM * NM * NM;
-    constexpr int BLOCK = HexCfg<NQ>::BLOCK, PER = (HexCfg<NQ>::EPB * M + BLOCK - 1) / BLOCK;
+    constexpr int BLOCK = C::BLOCK, PER = (C::EPB * M + BLOCK - 1) / BLOCK;
     int gi[PER];
     signed char sg[PER];
 #pragma unroll
@@ -109,7 +109,7 @@ __device__ __forceinline__ void load_modes_block_gather(const T *__restrict__ gl
 
 // Block-cooperative, fully coalesced store of nv elements' coefficients from the padded
 // pencil buffers buf(slot) to dst.
-template <int NM, int NQ, typename T, typename BufFn>
+template <int NM, int NQ, typename C, typename T, typename BufFn>
 __device__ __forceinline__ void store_modes_block(T *__restrict__ dst, int nv, BufFn buf)
 {
     constexpr int M = NM * NM * NM;
@@ -122,50 +122,53 @@ __device__ __forceinline__ void store_modes_block(T *__restrict__ dst, int nv, B
 
 // Mode pencils -> u (registers, k-column of thread (i,j)).  pencil(p) returns the p-th
 // coefficient of this thread's p-pencil (t = r*NM + q); uses buf0 and buf1.
-template <int NM, int NQ, typename T, typename PencilFn>
+template <int NM, int NQ, typename T, bool AGAIN = true, typename PencilFn>
 __device__ __forceinline__ void hex_bwd_to_columns(const Tab<NM, NQ, T> &tab, PencilFn pencil,
                                                    bool active, int t, T *buf0, T *buf1,
                                                    T (&u)[NQ])
 {
     // p -> i on p-pencils (thread (q, r))
     if (active && t < NM * NM) {
+        const auto &tb = reread<AGAIN>(tab);
         T uh[NM];
 #pragma unroll
         for (int p = 0; p < NM; ++p) uh[p] = pencil(p);
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
-            T s = uh[0] * tab.B[i];
+            T s = uh[0] * tb.B[i];
 #pragma unroll
-            for (int p = 1; p < NM; ++p) s = fma(uh[p], tab.B[p * NQ + i], s);
+            for (int p = 1; p < NM; ++p) s = fma(uh[p], tb.B[p * NQ + i], s);
             buf0[t * NQ + i] = s;  // s1[r][q][i], t = r*NM + q
         }
     }
     __syncthreads();
     // q -> j on q-pencils (thread (i, r))
     if (active && t < NQ * NM) {
+        const auto &tb = reread<AGAIN>(tab);
         const int i = t % NQ, r = t / NQ;
         T s1[NM];
 #pragma unroll
         for (int q = 0; q < NM; ++q) s1[q] = buf0[(r * NM + q) * NQ + i];
 #pragma unroll
         for (int j = 0; j < NQ; ++j) {
-            T s = s1[0] * tab.B[j];
+            T s = s1[0] * tb.B[j];
 #pragma unroll
-            for (int q = 1; q < NM; ++q) s = fma(s1[q], tab.B[q * NQ + j], s);
+            for (int q = 1; q < NM; ++q) s = fma(s1[q], tb.B[q * NQ + j], s);
             buf1[(r * NQ + j) * NQ + i] = s;  // s2[r][j][i]
         }
     }
     __syncthreads();
     // r -> k on r-pencils (thread (i, j)): the element's k-columns
     if (active) {
+        const auto &tb = reread<AGAIN>(tab);
         T s2[NM];
 #pragma unroll
         for (int r = 0; r < NM; ++r) s2[r] = buf1[r * NQ * NQ + t];
 #pragma unroll
         for (int k = 0; k < NQ; ++k) {
-            T s = s2[0] * tab.B[k];
+            T s = s2[0] * tb.B[k];
 #pragma unroll
-            for (int r = 1; r < NM; ++r) s = fma(s2[r], tab.B[r * NQ + k], s);
+            for (int r = 1; r < NM; ++r) s = fma(s2[r], tb.B[r * NQ + k], s);
             u[k] = s;
         }
     } else {
@@ -177,47 +180,50 @@ __device__ __forceinline__ void hex_bwd_to_columns(const Tab<NM, NQ, T> &tab, Pe
 // k-columns acc (registers of thread (i,j)) -> (B x B x B)^T acc; emit(p, v) receives the
 // p-th coefficient of this thread's p-pencil (t = r*NM + q).  Uses buf0 and buf1; emit may
 // write to buf0.
-template <int NM, int NQ, typename T, typename EmitFn>
+template <int NM, int NQ, typename T, bool AGAIN = true, typename EmitFn>
 __device__ __forceinline__ void hex_columns_to_modes(const Tab<NM, NQ, T> &tab,
                                                      const T (&acc)[NQ], bool active, int t,
                                                      T *buf0, T *buf1, EmitFn emit)
 {
     // k -> r in registers
     if (active) {
+        const auto &tb = reread<AGAIN>(tab);
 #pragma unroll
         for (int r = 0; r < NM; ++r) {
-            T s = acc[0] * tab.B[r * NQ];
+            T s = acc[0] * tb.B[r * NQ];
 #pragma unroll
-            for (int k = 1; k < NQ; ++k) s = fma(acc[k], tab.B[r * NQ + k], s);
+            for (int k = 1; k < NQ; ++k) s = fma(acc[k], tb.B[r * NQ + k], s);
             buf0[r * NQ * NQ + t] = s;  // z2[r][j][i]
         }
     }
     __syncthreads();
     // j -> q on j-pencils (thread (i, r))
     if (active && t < NQ * NM) {
+        const auto &tb = reread<AGAIN>(tab);
         const int i = t % NQ, r = t / NQ;
         T v[NQ];
 #pragma unroll
         for (int j = 0; j < NQ; ++j) v[j] = buf0[(r * NQ + j) * NQ + i];
 #pragma unroll
         for (int q = 0; q < NM; ++q) {
-            T s = v[0] * tab.B[q * NQ];
+            T s = v[0] * tb.B[q * NQ];
 #pragma unroll
-            for (int j = 1; j < NQ; ++j) s = fma(v[j], tab.B[q * NQ + j], s);
+            for (int j = 1; j < NQ; ++j) s = fma(v[j], tb.B[q * NQ + j], s);
             buf1[(r * NM + q) * NQ + i] = s;  // z1[r][q][i]
         }
     }
     __syncthreads();
     // i -> p on i-pencils (thread (q, r))
     if (active && t < NM * NM) {
+        const auto &tb = reread<AGAIN>(tab);
         T v[NQ];
 #pragma unroll
         for (int i = 0; i < NQ; ++i) v[i] = buf1[t * NQ + i];
 #pragma unroll
         for (int p = 0; p < NM; ++p) {
-            T s = v[0] * tab.B[p * NQ];
+            T s = v[0] * tb.B[p * NQ];
 #pragma unroll
-            for (int i = 1; i < NQ; ++i) s = fma(v[i], tab.B[p * NQ + i], s);
+            for (int i = 1; i < NQ; ++i) s = fma(v[i], tb.B[p * NQ + i], s);
             emit(p, s);
         }
     }
@@ -275,7 +281,8 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_bwdtrans_kernel(
 }
 
 // IProductWRTBase: out = (B x B x B)^T diag(w J) f.  GEO = kUnit gives the Euclidean
-// transpose of BwdTrans (w J == 1).
+// transpose of BwdTrans (w J == 1).  The tables stay with the compiler: read again, deformed
+// took 107 us for 80 with 8 modes and 9 points (12e6 points), 66 for 51 with 6 and 7.
 template <int NM, int NQ, typename T, int GEO>
 __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_iproduct_kernel(
     const Tab<NM, NQ, T> tab, int nElmt, const T *__restrict__ in,
@@ -313,7 +320,7 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_iproduct_kernel(
         for (int k = 0; k < NQ; ++k) acc[k] = T(0);
     }
     T *dst = out + e * M + t * NM;
-    hex_columns_to_modes<NM, NQ, T>(
+    hex_columns_to_modes<NM, NQ, T, false>(
         tab, acc, active, t, lds[es][0], lds[es][1], [&](int p, T v) {
             if (valid) st_stream(dst + p, v);
         });
@@ -323,13 +330,15 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_iproduct_kernel(
 // of the reference's MassMatrixOp_MatFree (StdRegions/StdExpansion.cpp:647-661:
 // BwdTrans, then IProductWRTBase).  The thread's geometry column (NQ values of w J) is
 // read once and reused for every vector, so each further vector streams only its
-// coefficients in and out.
+// coefficients in and out.  From 8 points the tables are read again (12e6 points, held /
+// read again: 8,9 132/78 us, 8,10 114/49, 6,8 43/29; 5,7 27/30, 4,6 26/28).
 template <int NM, int NQ, typename T, int GEO>
 __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_mass_kernel(
     const Tab<NM, NQ, T> tab, int nElmt, int nvec, const T *__restrict__ in, long ldin,
     const T *__restrict__ geom, T *__restrict__ out, long ldout)
 {
     using C = HexCfg<NQ>;
+    constexpr bool AGAIN = NQ >= 8;
     constexpr int M = NM * NM * NM, Q = NQ * NQ * NQ;
     __shared__ T lds[C::EPB][2][Q];
     const int eb = threadIdx.x / C::TPE;
@@ -366,12 +375,12 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_mass_kernel(
             for (int p = 0; p < NM; ++p) uh[p] = T(0);
         }
         T u[NQ];
-        hex_bwd_to_columns<NM, NQ, T>(tab, [&](int p) { return uh[p]; }, active, t,
+        hex_bwd_to_columns<NM, NQ, T, AGAIN>(tab, [&](int p) { return uh[p]; }, active, t,
                                       lds[es][0], lds[es][1], u);
 #pragma unroll
         for (int k = 0; k < NQ; ++k) u[k] *= jw[k];
         T *dst = out + v * ldout + e * M + t * NM;
-        hex_columns_to_modes<NM, NQ, T>(
+        hex_columns_to_modes<NM, NQ, T, AGAIN>(
             tab, u, active, t, lds[es][0], lds[es][1], [&](int p, T x) {
                 if (valid) st_stream(dst + p, x);
             });
@@ -409,15 +418,33 @@ constexpr int helm_geo_prefetch()
     return per > 56 ? 0 : (56 / per > 7 ? 7 : 56 / per);
 }
 
+// Whether a launch packs elements into 256-thread workgroups (HexCfg).  Measured at 12e6
+// points, nq - 1 modes, narrow / wide in us: 6 points FP64 regular 98/74, deformed 152/137;
+// 9 points 123/110, 205/183; 7 points FP32 regular 57/50, but FP64 133/150 deformed; 6 points
+// FP32 regular 64/47, deformed 74/79; 5 points FP64 70/70, 121/127.  BwdTrans, IProduct and
+// PhysDeriv, bound by HBM, gain nothing (7 points: IProduct 51/70, PhysDeriv 76/101).
+template <int NQ, typename T, int GEO, bool MANY>
+constexpr bool helm_wide()
+{
+    if (MANY) return false;  // the geometry staged in LDS takes the room
+    constexpr bool f64 = sizeof(T) == 8;
+    if (NQ == 6) return f64 || GEO != kDeformed;
+    if (NQ == 7) return !f64 && GEO != kDeformed;
+    return NQ == 9;
+}
+
+template <int NQ, typename T, int GEO, bool MANY>
+using HelmCfg = HexCfg<NQ, helm_wide<NQ, T, GEO, MANY>()>;
+
 template <int NM, int NQ, typename T, int GEO, bool GATHER = false, bool MANY = false>
-__global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_helmholtz_kernel(
+__global__ __launch_bounds__((HelmCfg<NQ, T, GEO, MANY>::BLOCK)) void hex_helmholtz_kernel(
     const Tab<NM, NQ, T> tab, int nElmt, T lambda, const T *__restrict__ in,
     const T *__restrict__ geom, T *__restrict__ out, const int *__restrict__ gmap = nullptr,
     const signed char *__restrict__ gsign = nullptr, int nvec = 1, long ldin = 0,
     long ldout = 0, const int *__restrict__ skip = nullptr)
 {
     if (GATHER && skip && *skip) return;
-    using C = HexCfg<NQ>;
+    using C = HelmCfg<NQ, T, GEO, MANY>;
     using Lb = HexLds<NM, NQ>;
     constexpr int M = Lb::M, Q = Lb::Q, TPE = C::TPE;
     constexpr long GS = geo_stride(7 * Q, sizeof(T));
@@ -466,10 +493,10 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_helmholtz_kernel(
 
     // 1. BwdTrans into k-columns; keep a copy of u in LDS for the cross derivatives.
     if constexpr (GATHER)
-        load_modes_block_gather<NM, NQ, T>(in, gmap + e0 * M, gsign + e0 * M, nv,
+        load_modes_block_gather<NM, NQ, C, T>(in, gmap + e0 * M, gsign + e0 * M, nv,
                                            [&](int sl) { return lds[sl][2]; });
     else
-        load_modes_block<NM, NQ, T>(in + e0 * M, nv, [&](int sl) { return lds[sl][2]; });
+        load_modes_block<NM, NQ, C, T>(in + e0 * M, nv, [&](int sl) { return lds[sl][2]; });
     __syncthreads();
     T u[NQ];
     hex_bwd_to_columns<NM, NQ, T>(
@@ -485,6 +512,7 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_helmholtz_kernel(
     // thread (j,k) = (t%NQ, t/NQ), d1 on j-pencils of thread (i,k) = (t%NQ, t/NQ),
     // d2 on this thread's k-column.
     if (active) {
+        const auto &tb = reread(tab);
         T v[NQ];
         {
             const int pj = t % NQ, pk = t / NQ;
@@ -492,21 +520,22 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_helmholtz_kernel(
             for (int l = 0; l < NQ; ++l) v[l] = buf2[(pk * NQ + pj) * NQ + l];
 #pragma unroll
             for (int i = 0; i < NQ; ++i) {
-                T s = v[0] * tab.D[i];
+                T s = v[0] * tb.D[i];
 #pragma unroll
-                for (int l = 1; l < NQ; ++l) s = fma(v[l], tab.D[l * NQ + i], s);
+                for (int l = 1; l < NQ; ++l) s = fma(v[l], tb.D[l * NQ + i], s);
                 buf0[(pk * NQ + pj) * NQ + i] = s;
             }
         }
         {
+            const auto &tb = reread(tab);
             const int pi = t % NQ, pk = t / NQ;
 #pragma unroll
             for (int l = 0; l < NQ; ++l) v[l] = buf2[(pk * NQ + l) * NQ + pi];
 #pragma unroll
             for (int j = 0; j < NQ; ++j) {
-                T s = v[0] * tab.D[j];
+                T s = v[0] * tb.D[j];
 #pragma unroll
-                for (int l = 1; l < NQ; ++l) s = fma(v[l], tab.D[l * NQ + j], s);
+                for (int l = 1; l < NQ; ++l) s = fma(v[l], tb.D[l * NQ + j], s);
                 buf1[(pk * NQ + j) * NQ + pi] = s;
             }
         }
@@ -514,13 +543,15 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_helmholtz_kernel(
     __syncthreads();
 
     // 3. Pointwise metric contraction and mass term on this thread's column.
+    const T wij = GEO == kRegular ? reread(tab).w[ci] * reread(tab).w[cj] : T(0);
+    const auto &tb = reread(tab);
     T g0[NQ], g1[NQ], g2[NQ], acc[NQ];
     if (valid) {
 #pragma unroll
         for (int k = 0; k < NQ; ++k) {
-            T d2 = u[0] * tab.D[k];
+            T d2 = u[0] * tb.D[k];
 #pragma unroll
-            for (int l = 1; l < NQ; ++l) d2 = fma(u[l], tab.D[l * NQ + k], d2);
+            for (int l = 1; l < NQ; ++l) d2 = fma(u[l], tb.D[l * NQ + k], d2);
             const T d0 = buf0[k * TPE + t];
             const T d1 = buf1[k * TPE + t];
             T jw, m00, m01, m02, m11, m12, m22;
@@ -553,7 +584,7 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_helmholtz_kernel(
                 m12 = ld_stream(g + 5 * Q);
                 m22 = ld_stream(g + 6 * Q);
             } else {
-                const T wq = tab.w[ci] * tab.w[cj] * tab.w[k];
+                const T wq = wij * tb.w[k];
                 const T *g = geom + e * 7;
                 jw = g[0] * wq;
                 m00 = g[1] * wq;
@@ -581,11 +612,12 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_helmholtz_kernel(
         }
     }
     // D^T along k in registers.
+    const auto &td = reread(tab);
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
         T s = acc[k];
 #pragma unroll
-        for (int l = 0; l < NQ; ++l) s = fma(g2[l], tab.D[k * NQ + l], s);
+        for (int l = 0; l < NQ; ++l) s = fma(g2[l], td.D[k * NQ + l], s);
         acc[k] = s;
     }
     __syncthreads();
@@ -593,29 +625,31 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_helmholtz_kernel(
     // 4. D^T along i (pencils of thread (j,k)) into buf2, then D^T along j (pencils of
     // thread (i,k)) added to it: three buffers instead of four per element.
     if (active) {
+        const auto &tb = reread(tab);
         T v[NQ];
         const int pj = t % NQ, pk = t / NQ;
 #pragma unroll
         for (int l = 0; l < NQ; ++l) v[l] = buf0[(pk * NQ + pj) * NQ + l];
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
-            T s = v[0] * tab.D[i * NQ];
+            T s = v[0] * tb.D[i * NQ];
 #pragma unroll
-            for (int l = 1; l < NQ; ++l) s = fma(v[l], tab.D[i * NQ + l], s);
+            for (int l = 1; l < NQ; ++l) s = fma(v[l], tb.D[i * NQ + l], s);
             buf2[(pk * NQ + pj) * NQ + i] = s;
         }
     }
     __syncthreads();
     if (active) {
+        const auto &tb = reread(tab);
         T v[NQ];
         const int pi = t % NQ, pk = t / NQ;
 #pragma unroll
         for (int l = 0; l < NQ; ++l) v[l] = buf1[(pk * NQ + l) * NQ + pi];
 #pragma unroll
         for (int j = 0; j < NQ; ++j) {
-            T s = v[0] * tab.D[j * NQ];
+            T s = v[0] * tb.D[j * NQ];
 #pragma unroll
-            for (int l = 1; l < NQ; ++l) s = fma(v[l], tab.D[j * NQ + l], s);
+            for (int l = 1; l < NQ; ++l) s = fma(v[l], tb.D[j * NQ + l], s);
             buf2[(pk * NQ + j) * NQ + pi] += s;
         }
     }
@@ -629,7 +663,7 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_helmholtz_kernel(
     hex_columns_to_modes<NM, NQ, T>(tab, acc, active, t, buf0, buf1,
                                     [&](int p, T v) { buf2[t * (NM + 1) + p] = v; });
     __syncthreads();
-    store_modes_block<NM, NQ, T>(out + e0 * M, nv, [&](int sl) { return lds[sl][2]; });
+    store_modes_block<NM, NQ, C, T>(out + e0 * M, nv, [&](int sl) { return lds[sl][2]; });
   }
 }
 
@@ -753,6 +787,7 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_iprod_deriv_kernel(
     T g0[NQ], g1[NQ], g2[NQ];
     if (valid) {
         const int ci = t % NQ, cj = t / NQ;
+        const T wij = GEO == kRegular ? tab.w[ci] * tab.w[cj] : T(0);
 #pragma unroll
         for (int k = 0; k < NQ; ++k) {
             const long o = e * Q + k * TPE + t;
@@ -763,7 +798,7 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_iprod_deriv_kernel(
 #pragma unroll
                 for (int d = 0; d < 9; ++d) f[d] = ld_stream(geom + e * GS + d * Q + k * TPE + t);
             } else {
-                const T wq = tab.w[ci] * tab.w[cj] * tab.w[k];
+                const T wq = wij * tab.w[k];
 #pragma unroll
                 for (int d = 0; d < 9; ++d) f[d] = geom[e * 9 + d] * wq;
             }
@@ -826,7 +861,7 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_iprod_deriv_kernel(
         for (int k = 0; k < NQ; ++k) acc[k] += buf0[k * TPE + t] + buf1[k * TPE + t];
     }
     T *dst = out + e * M + t * NM;
-    hex_columns_to_modes<NM, NQ, T>(tab, acc, active, t, buf2, buf3, [&](int p, T v) {
+    hex_columns_to_modes<NM, NQ, T, false>(tab, acc, active, t, buf2, buf3, [&](int p, T v) {
         if (valid) st_stream(dst + p, v);
     });
 }

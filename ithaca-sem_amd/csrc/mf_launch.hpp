@@ -26,9 +26,11 @@ hipError_t launch_hex(const LaunchArgs &a)
     const T *geom = static_cast<const T *>(a.geom);
     T *out = static_cast<T *>(a.out);
     if constexpr (KIND == kHelmholtz) {
+        using W = HelmCfg<NQ, T, GEO, false>;
+        const dim3 wgrid((unsigned)((a.nElmt + W::EPB - 1) / W::EPB)), wblock(W::BLOCK);
         if constexpr (std::is_same_v<T, double>) {
             if (a.gmap) {
-                hex_helmholtz_kernel<NM, NQ, T, GEO, true><<<grid, block, 0, a.stream>>>(
+                hex_helmholtz_kernel<NM, NQ, T, GEO, true><<<wgrid, wblock, 0, a.stream>>>(
                     tab, a.nElmt, T(a.lambda), in, geom, out, a.gmap, a.gsign, 1, 0, 0, a.skip);
                 return hipGetLastError();
             }
@@ -41,7 +43,7 @@ hipError_t launch_hex(const LaunchArgs &a)
             return hipGetLastError();
         }
         hex_helmholtz_kernel<NM, NQ, T, GEO>
-            <<<grid, block, 0, a.stream>>>(tab, a.nElmt, T(a.lambda), in, geom, out);
+            <<<wgrid, wblock, 0, a.stream>>>(tab, a.nElmt, T(a.lambda), in, geom, out);
     } else if constexpr (KIND == kMass) {
         hex_mass_kernel<NM, NQ, T, GEO><<<grid, block, 0, a.stream>>>(
             tab, a.nElmt, a.nvec, in, a.ldin, geom, out, a.ldout);

@@ -16,12 +16,13 @@
 namespace imf {
 
 // u_hat (global) -> u (registers: thread i holds u[j] at point (i, j)).  Uses buf0.
-template <int NM, int NQ, typename T>
+template <int NM, int NQ, typename T, bool AGAIN = true>
 __device__ __forceinline__ void quad_bwd_to_lines(const Tab<NM, NQ, T> &tab,
                                                   const T *__restrict__ src, bool valid,
                                                   bool active, int t, T *buf0, T (&u)[NQ])
 {
     if (active && t < NM) {
+        const auto &tb = reread<AGAIN>(tab);
         T uh[NM];
         if (valid) {
 #pragma unroll
@@ -32,22 +33,23 @@ __device__ __forceinline__ void quad_bwd_to_lines(const Tab<NM, NQ, T> &tab,
         }
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
-            T s = uh[0] * tab.B[i];
+            T s = uh[0] * tb.B[i];
 #pragma unroll
-            for (int p = 1; p < NM; ++p) s = fma(uh[p], tab.B[p * NQ + i], s);
+            for (int p = 1; p < NM; ++p) s = fma(uh[p], tb.B[p * NQ + i], s);
             buf0[t * NQ + i] = s;  // s1[q][i]
         }
     }
     __syncthreads();
     if (active) {
+        const auto &tb = reread<AGAIN>(tab);
         T s1[NM];
 #pragma unroll
         for (int q = 0; q < NM; ++q) s1[q] = buf0[q * NQ + t];
 #pragma unroll
         for (int j = 0; j < NQ; ++j) {
-            T s = s1[0] * tab.B[j];
+            T s = s1[0] * tb.B[j];
 #pragma unroll
-            for (int q = 1; q < NM; ++q) s = fma(s1[q], tab.B[q * NQ + j], s);
+            for (int q = 1; q < NM; ++q) s = fma(s1[q], tb.B[q * NQ + j], s);
             u[j] = s;
         }
     } else {
@@ -58,30 +60,32 @@ __device__ __forceinline__ void quad_bwd_to_lines(const Tab<NM, NQ, T> &tab,
 
 // acc (registers, j-line of thread i) -> out = (B x B)^T acc.  Uses buf0; the caller
 // must have synchronised any earlier readers of buf0.
-template <int NM, int NQ, typename T>
+template <int NM, int NQ, typename T, bool AGAIN = true>
 __device__ __forceinline__ void quad_lines_to_modes(const Tab<NM, NQ, T> &tab,
                                                     const T (&acc)[NQ], T *__restrict__ dst,
                                                     bool valid, bool active, int t, T *buf0)
 {
     if (active) {
+        const auto &tb = reread<AGAIN>(tab);
 #pragma unroll
         for (int q = 0; q < NM; ++q) {
-            T s = acc[0] * tab.B[q * NQ];
+            T s = acc[0] * tb.B[q * NQ];
 #pragma unroll
-            for (int j = 1; j < NQ; ++j) s = fma(acc[j], tab.B[q * NQ + j], s);
+            for (int j = 1; j < NQ; ++j) s = fma(acc[j], tb.B[q * NQ + j], s);
             buf0[q * NQ + t] = s;  // z[q][i]
         }
     }
     __syncthreads();
     if (active && t < NM && valid) {
+        const auto &tb = reread<AGAIN>(tab);
         T v[NQ];
 #pragma unroll
         for (int i = 0; i < NQ; ++i) v[i] = buf0[t * NQ + i];
 #pragma unroll
         for (int p = 0; p < NM; ++p) {
-            T s = v[0] * tab.B[p * NQ];
+            T s = v[0] * tb.B[p * NQ];
 #pragma unroll
-            for (int i = 1; i < NQ; ++i) s = fma(v[i], tab.B[p * NQ + i], s);
+            for (int i = 1; i < NQ; ++i) s = fma(v[i], tb.B[p * NQ + i], s);
             st_stream(dst + t * NM + p, s);
         }
     }
@@ -152,7 +156,7 @@ __global__ __launch_bounds__(QuadCfg<NQ>::BLOCK) void quad_iproduct_kernel(
 #pragma unroll
         for (int j = 0; j < NQ; ++j) acc[j] = T(0);
     }
-    quad_lines_to_modes<NM, NQ, T>(tab, acc, out + e * M, valid, active, t, lds[es]);
+    quad_lines_to_modes<NM, NQ, T, false>(tab, acc, out + e * M, valid, active, t, lds[es]);
 }
 
 // Packed geometry: deformed [e][4][Q] (Jw, JwG00, JwG01, JwG11); regular [e][4]
@@ -163,6 +167,7 @@ __global__ __launch_bounds__(QuadCfg<NQ>::BLOCK) void quad_helmholtz_kernel(
     const T *__restrict__ geom, T *__restrict__ out)
 {
     using C = QuadCfg<NQ>;
+    constexpr bool AGAIN = NQ >= 9;  // 6,8 deformed at 12e6 points: held 77 us, read again 80
     constexpr int M = NM * NM, Q = NQ * NQ;
     __shared__ T lds[C::EPB][2][Q];
     const int eb = threadIdx.x / C::TPE;
@@ -174,7 +179,7 @@ __global__ __launch_bounds__(QuadCfg<NQ>::BLOCK) void quad_helmholtz_kernel(
     T *buf0 = lds[es][0], *buf1 = lds[es][1];
 
     T u[NQ];
-    quad_bwd_to_lines<NM, NQ, T>(tab, in + e * M, valid, active, t, buf0, u);
+    quad_bwd_to_lines<NM, NQ, T, AGAIN>(tab, in + e * M, valid, active, t, buf0, u);
     if (active) {
 #pragma unroll
         for (int j = 0; j < NQ; ++j) buf1[j * NQ + t] = u[j];
@@ -182,26 +187,28 @@ __global__ __launch_bounds__(QuadCfg<NQ>::BLOCK) void quad_helmholtz_kernel(
     __syncthreads();
     // d0 on i-lines of thread j = t
     if (active) {
+        const auto &tb = reread<AGAIN>(tab);
         T v[NQ];
 #pragma unroll
         for (int l = 0; l < NQ; ++l) v[l] = buf1[t * NQ + l];
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
-            T s = v[0] * tab.D[i];
+            T s = v[0] * tb.D[i];
 #pragma unroll
-            for (int l = 1; l < NQ; ++l) s = fma(v[l], tab.D[l * NQ + i], s);
+            for (int l = 1; l < NQ; ++l) s = fma(v[l], tb.D[l * NQ + i], s);
             buf0[t * NQ + i] = s;
         }
     }
     __syncthreads();
     T g0[NQ], g1[NQ], acc[NQ];
     if (valid) {
-        const T wi = tab.w[t];
+        const auto &tb = reread<AGAIN>(tab);
+        const T wi = tb.w[t];
 #pragma unroll
         for (int j = 0; j < NQ; ++j) {
-            T d1 = u[0] * tab.D[j];
+            T d1 = u[0] * tb.D[j];
 #pragma unroll
-            for (int l = 1; l < NQ; ++l) d1 = fma(u[l], tab.D[l * NQ + j], d1);
+            for (int l = 1; l < NQ; ++l) d1 = fma(u[l], tb.D[l * NQ + j], d1);
             const T d0 = buf0[j * NQ + t];
             T jw, m00, m01, m11;
             if (GEO == kDeformed) {
@@ -211,7 +218,7 @@ __global__ __launch_bounds__(QuadCfg<NQ>::BLOCK) void quad_helmholtz_kernel(
                 m01 = ld_stream(g + 2 * Q);
                 m11 = ld_stream(g + 3 * Q);
             } else {
-                const T wq = wi * tab.w[j];
+                const T wq = wi * tb.w[j];
                 const T *g = geom + e * 4;
                 jw = g[0] * wq;
                 m00 = g[1] * wq;
@@ -230,23 +237,25 @@ __global__ __launch_bounds__(QuadCfg<NQ>::BLOCK) void quad_helmholtz_kernel(
 #pragma unroll
         for (int j = 0; j < NQ; ++j) buf1[j * NQ + t] = g0[j];
     }
+    const auto &td = reread<AGAIN>(tab);
 #pragma unroll
     for (int j = 0; j < NQ; ++j) {
         T s = acc[j];
 #pragma unroll
-        for (int l = 0; l < NQ; ++l) s = fma(g1[l], tab.D[j * NQ + l], s);
+        for (int l = 0; l < NQ; ++l) s = fma(g1[l], td.D[j * NQ + l], s);
         acc[j] = s;
     }
     __syncthreads();
     if (active) {
+        const auto &tb = reread<AGAIN>(tab);
         T v[NQ];
 #pragma unroll
         for (int l = 0; l < NQ; ++l) v[l] = buf1[t * NQ + l];
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
-            T s = v[0] * tab.D[i * NQ];
+            T s = v[0] * tb.D[i * NQ];
 #pragma unroll
-            for (int l = 1; l < NQ; ++l) s = fma(v[l], tab.D[i * NQ + l], s);
+            for (int l = 1; l < NQ; ++l) s = fma(v[l], tb.D[i * NQ + l], s);
             buf0[t * NQ + i] = s;
         }
     }
@@ -394,7 +403,7 @@ __global__ __launch_bounds__(QuadCfg<NQ>::BLOCK) void quad_iprod_deriv_kernel(
         for (int j = 0; j < NQ; ++j) acc[j] += buf0[j * NQ + t];
     }
     __syncthreads();
-    quad_lines_to_modes<NM, NQ, T>(tab, acc, out + e * M, valid, active, t, buf1);
+    quad_lines_to_modes<NM, NQ, T, false>(tab, acc, out + e * M, valid, active, t, buf1);
 }
 
 }  // namespace imf

@@ -416,3 +416,32 @@ def test_reference_collection_lambda_zero_cases(nq):
     ref[np.abs(ref) < 1e-14] = 0.0
     close = np.abs(got - ref) <= 1e-10 * np.minimum(np.abs(got), np.abs(ref))  # the strong form
     assert np.all(close), np.abs(got - ref).max()
+
+
+@pytest.mark.parametrize("E", [1, 8, 65])
+@pytest.mark.parametrize("shape,nm,nq", [("quad", 5, 9), ("quad", 7, 8), ("quad", 8, 10),
+                                         ("hex", 5, 6), ("hex", 6, 7), ("hex", 5, 9),
+                                         ("hex", 7, 8), ("hex", 8, 10)])
+def test_helmholtz_and_mass_tables(shape, nm, nq, E):
+    """On both sides of the orders from which the kernels read their tables again at each stage
+    and pack elements into 256 threads (7, 5 and 3 of them)."""
+    print(f"[case] {shape} nm={nm} nq={nq} E={E}", flush=True)
+    rng = np.random.default_rng(nq + E)
+    dim = 3 if shape == "hex" else 2
+    verts = (mesh.hex_box if dim == 3 else mesh.quad_box)(1, 0.0, rng) * rng.uniform(0.5, 2.0, (E, 1, 1))
+    b = O.basis(nm, nq)
+    for deformed in (False, True):
+        v = verts + (0.1 * rng.uniform(-1, 1, verts.shape) if deformed else 0.0)
+        jac, df = (O.geom_hex if dim == 3 else O.geom_quad)(v, nq, b["z"], deformed)
+        u = rng.uniform(-1, 1, E * nm ** dim)
+        geo = f"{shape.capitalize()}_{'Deformed' if deformed else 'Regular'}"
+        op = _op(f"Helmholtz_{geo}", nm, nq, E, b, jac, df)
+        op.set_lambda(2.5)
+        want = O.helmholtz(shape, b, E, deformed, jac, df, 2.5, u)
+        assert rel(op.apply(_dev(u)).cpu().numpy(), want) < TOL64
+        op32 = _op(f"Helmholtz_{geo}", nm, nq, E, b, jac, df, prec=H.FP32)
+        op32.set_lambda(2.5)
+        assert rel(op32.apply(_dev(u, torch.float32)).double().cpu().numpy(), want) < TOL32 * 10
+        if dim == 3:
+            m = O.iproduct("hex", b, E, deformed, jac, O.bwdtrans("hex", b, E, u))
+            assert rel(_op(f"Mass_{geo}", nm, nq, E, b, jac).apply(_dev(u)).cpu().numpy(), m) < TOL64
