@@ -192,6 +192,14 @@ int imf_apply_transpose_device(imf_op op, const void *d_in, void *d_out, void *s
 int imf_apply_many_device(imf_op op, int nvec, const void *d_in, long ld_in, void *d_out,
                           long ld_out, void *stream);
 
+/* The weighted L2 misfit of a field and its residual: r = u - f, written over d_u, and
+ * *d_loss = 1/2 sum_q w_q r_q^2, over n values.  d_part holds IMF_MISFIT_PARTS doubles of
+ * scratch.  FP64 device arrays that do not overlap, asynchronous, allocates nothing; the sum's
+ * order is fixed.  No reference counterpart. */
+#define IMF_MISFIT_PARTS 2048
+int imf_misfit_device(size_t n, double *d_u, const double *d_f, const double *d_w, double *d_part,
+                      double *d_loss, void *stream);
+
 /* Message of the last failing call on this thread ("" if none). */
 const char *imf_last_error(void);
 

@@ -53,6 +53,7 @@ def lib():
         L.imf_apply_device.argtypes = [vp, vp, vp, vp]
         L.imf_apply_transpose_device.argtypes = [vp, vp, vp, vp]
         L.imf_apply_many_device.argtypes = [vp, i, vp, ctypes.c_long, vp, ctypes.c_long, vp]
+        L.imf_misfit_device.argtypes = [sz, vp, vp, vp, vp, vp, vp]
         L.imf_last_error.restype = ctypes.c_char_p
         L.imf_basis_modified_a.argtypes = [i, i, vp, vp, vp, vp, vp]
         L.imf_geom_hex_device.argtypes = [vp, i, i, vp, i, vp, vp, vp]

@@ -217,3 +217,26 @@ def test_helmsolve_adjoint_variable_order():
     assert np.linalg.norm(g[free] - w) <= 1e-9 * np.linalg.norm(w)
     gl = -w @ ((A3 - A)[free][:, free] @ u)
     assert abs(lam.grad.item() - gl) <= 1e-8 * abs(gl)
+
+
+@pytest.mark.parametrize("n", [0, 1, 2, 3, 511, 513, 2 * 256 * 2048 - 1, 2 * 256 * 2048 + 513])
+def test_misfit_sizes_and_forms(n):
+    """The one-pass residual and misfit at the ends of its grid, on aligned and misaligned
+    vectors, against the general path's forms and 64-bit sums (n roundings of 1e-16 at most,
+    in a tree: bar 1e-13)."""
+    from ithaca_hip.autograd import _residual_and_misfit
+    print(f"[case] misfit n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    u, f, w = rng.uniform(-1, 1, n), rng.uniform(-1, 1, n), rng.uniform(0.5, 2, n)
+    want = 0.5 * np.sum((w * (u - f) ** 2).astype(np.longdouble))
+
+    def shifted(a, k):
+        t = torch.zeros(n + 2, dtype=torch.float64, device="cuda")[k:k + n]
+        return t.copy_(_dev(a))
+
+    strided = torch.zeros((n, 2), dtype=torch.float64, device="cuda")[:, 0].copy_(_dev(f))
+    for tu, tf, tw in [(_dev(u), _dev(f), _dev(w)), (shifted(u, 1), _dev(f), _dev(w)),
+                       (_dev(u), shifted(f, 1), shifted(w, 1)), (_dev(u), strided, _dev(w))]:
+        r, loss = _residual_and_misfit(tu, tf, tw)
+        assert loss.shape == () and np.array_equal(r.cpu().numpy(), u - f)
+        assert abs(loss.item() - float(want)) <= 1e-13 * float(want)
