@@ -4,8 +4,8 @@
 // once, r written once, 32 B per point.  As a subtraction, a product and a dot product it read
 // and wrote 64 B: with the transforms around it, on 32 768 hexes with 343 points (11.2e6
 // points), a misfit and its gradient took 197 us so and take 149.  Each thread keeps its own
-// FP64 sum, a workgroup leaves one partial sum, and a
-// second kernel adds those in a fixed order, so the result does not vary from run to run.
+// FP64 sum, a workgroup leaves one partial sum, and a second kernel adds those in a fixed
+// order, so the result does not vary from run to run.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
