@@ -198,7 +198,8 @@ struct LuLds {
     int perm[NMAX];                // rows eliminated, in order, then the rows left
     unsigned ckey[2][NT / 64];
     int count[NT / 64];            // rows left by wave
-    int zero, inst;
+    int zero;                      // a pivot without a finite reciprocal (lu_divide: zero or NaN)
+    int inst;
 };
 __shared__ LuLds sh;  // of solve_fp64_kernel and the functions it calls
 
@@ -233,7 +234,8 @@ __device__ __forceinline__ unsigned pivot_key(bool act, double x)
 
 // 1 / p to within an ulp or two (v_rcp_f64 and two Newton steps; the callers' products are
 // corrected against p): the chain of a pivot column waits for it, and the correctly rounded
-// quotient takes twice as long.  Infinite or NaN for a zero, subnormal or non-finite p.
+// quotient takes twice as long.  Infinite or NaN for a zero, subnormal or non-finite p: an
+// instance that meets one is looked at again by lu_divide.
 __device__ __forceinline__ double fast_rcp(double p)
 {
     double r = __builtin_amdgcn_rcp(p);
@@ -584,6 +586,76 @@ __device__ __noinline__ double lu_back(GCPtr A, int ld, int n)
     return yi;
 }
 
+// An instance with a pivot that has no finite reciprocal.  When the first such pivot is zero or
+// NaN the matrix is singular: sh.zero stays set and x is returned.  A subnormal or infinite pivot
+// can be divided by: the instance is assembled and solved again, column by column (a wave per
+// row), with divisions; sh.zero then tells of a zero or NaN pivot.  Rare, so kept short and out
+// of the kernel's registers.
+__device__ __noinline__ double lu_divide(GPtr A, int ld, int n, int nq, GCPtr Ai, GCPtr th, GCPtr b,
+                                         int transpose, double x)
+{
+    constexpr int NW = NT / 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (tid == 0) sh.inst = n;
+    __syncthreads();
+    const double d = tid < n ? A[(long)sh.perm[tid] * ld + tid] : 1.0;
+    if (!(fabs(fast_rcp(d)) < INFINITY)) atomicMin(&sh.inst, tid);
+    __syncthreads();
+    const int first = sh.inst;
+    if (first >= n) return x;
+    if (tid == first) sh.zero = !(fabs(d) > 0.0);
+    __syncthreads();
+    if (sh.zero) return x;
+    for (int i = tid; i < n * n; i += NT) {
+        double s = 0.0;
+        for (int q = 0; q < nq; ++q) s += th[q] * Ai[(long)q * n * n + i];
+        const int r = i / n, c = i - r * n;
+        A[transpose ? (long)c * ld + r : (long)r * ld + c] = s;
+    }
+    if (tid < n) {
+        A[(long)tid * ld + n] = b[tid];
+        sh.perm[tid] = tid;
+    }
+    __syncthreads();
+    for (int c = 0; c < n; ++c) {
+        const int pos = c + tid;
+        double v = pos < n ? fabs(A[(long)sh.perm[pos] * ld + c]) : -1.0;
+        if (v != v) v = -1.0;  // NaN: never a pivot
+        const double top = wave_max(v);
+        const int pl = __builtin_ffsll((long long)__ballot(v == top)) - 1;
+        if (lane == pl) {
+            sh.cand[0][wave][0] = top;
+            sh.count[wave] = pos;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            int w = 0;
+            for (int k = 1; k < NW; ++k)
+                if (sh.cand[0][k][0] > sh.cand[0][w][0]) w = k;
+            if (!(sh.cand[0][w][0] > 0.0)) sh.zero = 1;
+            const int p = sh.cand[0][w][0] < 0.0 ? c : sh.count[w], r = sh.perm[p];
+            sh.perm[p] = sh.perm[c];
+            sh.perm[c] = r;
+        }
+        __syncthreads();
+        const GCPtr P = A + (long)sh.perm[c] * ld;
+        for (int i = c + 1 + wave; i < n; i += NW) {
+            const GPtr row = A + (long)sh.perm[i] * ld;
+            const double l = row[c] / P[c];
+            for (int j = c + 1 + lane; j <= n; j += 64) row[j] -= l * P[j];
+        }
+        __syncthreads();
+    }
+    const GCPtr row = A + (long)(tid < n ? sh.perm[tid] : 0) * ld;
+    double y = row[n];
+    for (int i = n - 1; i >= 0; --i) {
+        if (tid == i) sh.ys[i] = y = y / row[i];
+        __syncthreads();
+        if (tid < i) y -= row[i] * sh.ys[i];
+    }
+    return y;
+}
+
 __global__ __launch_bounds__(NT, 3) void solve_fp64_kernel(Args a)
 {
     const int tid = threadIdx.x;
@@ -662,7 +734,9 @@ __global__ __launch_bounds__(NT, 3) void solve_fp64_kernel(Args a)
             }
             __syncthreads();
         }
-        const double x = lu_back(A, ld, n);
+        double x = lu_back(A, ld, n);
+        if (__builtin_amdgcn_readfirstlane(sh.zero))
+            x = lu_divide(A, ld, n, nq, (GCPtr)Ai, (GCPtr)th, (GCPtr)(a.b + vo), a.transpose, x);
         const int st = sh.zero ? 1 : fallback ? 3 : 0;
         if (tid < n) a.x[vo + tid] = x;
         if (tid == 0) {

@@ -320,3 +320,47 @@ def test_fp64_solves_at_panel_edges(transpose):
         scale = np.array([np.abs(lam[sl]) @ (np.abs(M[q]) @ np.abs(x[sl])) for q in range(Q)])
         got = grad[batch.t_off[i]:batch.t_off[i] + Q]
         assert np.abs(got - ref).max() < 1e-14 * n * scale.max()
+
+
+@pytest.mark.parametrize("transpose", [False, True])
+def test_fp64_solves_with_pivots_beyond_the_reciprocal(transpose):
+    """Pivots that are subnormal, very small, very large or infinite are divided by.  A = R diag(s)
+    with R of 8-bit entries plus a dominant diagonal and s = 1 except in one column: its entries
+    are exact also where they are subnormal.  Bar: backward error on R (y = s x), 4 n eps, plus
+    n 2^-24 where the column is subnormal (at 2^-1050 an entry keeps 24 bits below one).  An
+    infinite diagonal entry gives x = 0 there."""
+    rng = np.random.default_rng(5)
+    cases = [(n, e, int(c * (n - 1))) for n in (1, 5, 16, 40, 70, 130, 256) for e in (-1050, -960, 960)
+             for c in (0.0, 0.6, 1.0)]
+    sizes = [n for n, _, _ in cases] + [20, 150]
+    batch = rom.Batch(sizes, [1] * len(sizes))
+    mats, rhs, Rs, ss = [], [], [], []
+    for n, e, c in cases:
+        M = np.round(rng.standard_normal((n, n)) * 256) / 256 + 4 * np.sqrt(n) // 1 * np.eye(n) + np.eye(n)
+        s = np.ones(n)
+        s[c] = 2.0 ** e
+        Rs.append(M)
+        ss.append(s)
+        mats.append((M * s).T if transpose else M * s)
+        rhs.append(rng.standard_normal(n) * (2.0 ** -200 if e < 0 else 1.0))  # x representable
+    for n in sizes[len(cases):]:
+        d = rng.uniform(1, 2, n)
+        d[n // 2] = np.inf
+        mats.append(np.diag(d))
+        rhs.append(rng.standard_normal(n))
+    status = torch.full((batch.n,), -1, dtype=torch.int32, device="cuda")
+    theta = torch.ones(batch.t_size, dtype=torch.float64, device="cuda")
+    x = batch.solve(_dev(np.concatenate([m.ravel() for m in mats])), theta, _dev(np.concatenate(rhs)),
+                    transpose=transpose, status=status).cpu().numpy()
+    st = status.cpu().numpy()
+    for i, n in enumerate(sizes):
+        xi, b = x[batch.v_off[i]:batch.v_off[i] + n], rhs[i]
+        assert st[i] == 0 and np.all(np.isfinite(xi)), (i, n, st[i])
+        if i >= len(cases):
+            d = np.diag(mats[i])
+            assert xi[n // 2] == 0 and np.allclose(xi, b / d, rtol=1e-15, atol=0)
+            continue
+        y = xi * ss[i]
+        back = np.abs(b - Rs[i] @ y).max() / (np.abs(Rs[i]).sum(1).max() * np.abs(y).max() + np.abs(b).max())
+        bar = 4 * max(n, 4) * 2.2e-16 + (n * 2.0 ** -24 if cases[i][1] == -1050 else 0.0)
+        assert back < bar, (cases[i], back)
