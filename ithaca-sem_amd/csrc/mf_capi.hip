@@ -21,6 +21,7 @@
 #include "mf_geom.hpp"
 #include "mf_launch.hpp"
 #include "mf_op.hpp"
+#include "mf_routes.hpp"
 #include "mf_seg.hpp"
 
 namespace {
@@ -327,28 +328,19 @@ void find_pencil(imf_op op, const double *const *bdata, const double *const *dbd
         op->pencil[1] = lookup(op->kind == imf::kBwdTrans ? imf::kIProduct : imf::kBwdTrans, m, q0);
 }
 
-// Dense products against the other kernels.  A dense product costs its matrix's entries per
-// element, a pencil kernel about the number of points.  Times in us at 12e6 points (at most
-// 120 000 elements), one point more than modes, dense / pencils, of 2 3 4 5 6 7 8 modes:
-//   Helmholtz  tetrahedra   9/20  14/48  31/98  45/152  48/177  72/207  144/242
-//              prisms       9/23  30/47  67/96  133/97  222/109  -/149  -/149
-//              pyramids     9/23  14/47  38/103 73/104  114/115  -/157  -/206
-//     (two points more: prisms of 5 and 6 modes 83/100, 150/133; pyramids of 6 80/112)
-//   BwdTrans   tetrahedra   9/8   16/20  27/33  51/53   52/50    78/66  101/69
-//              prisms      12/9   17/21  56/36  77/45  101/44   127/53  165/57
-//              pyramids    12/9   17/19  39/36  60/46   79/45   108/63  139/76
-//   IProduct   tetrahedra   8/9   13/25  28/54  39/79   41/74   57/106   97/109
-//              prisms       8/12  20/24  43/47  58/61  100/59   137/72  163/74
-//              pyramids     8/12  14/24  35/49  50/64   80/65   103/106 160/116
-// Without a pencil kernel (triangles, other point counts) the alternative is the runtime-size
-// kernel, which only a prism's transform to the points with 30 000 entries or more meets
-// (6 / 7 / 8 modes: 99 / 102 / 141 us).
 bool dense_pays(const imf_op op, int tr, bool helm, bool from_modes)
 {
-    const long M = (long)op->M, Q = (long)op->Q;
-    if (!op->pencil[tr]) return helm || !from_modes || op->shape != imf::kPrism || M * Q <= 30000;
-    if (helm) return M * M < 27 * Q;
-    return from_modes ? M <= 20 : op->shape == imf::kTet || M <= 80;
+    imf::DenseCase c{};
+    c.shape = op->shape == imf::kTri ? imf::kRouteTri : op->shape == imf::kTet ? imf::kRouteTet
+            : op->shape == imf::kPrism ? imf::kRoutePrism : imf::kRoutePyr;
+    c.helm = helm;
+    c.from_modes = from_modes;
+    c.point_scale = op->kind == imf::kIProduct && op->deformed && !from_modes;
+    c.pencil = op->pencil[tr] != nullptr;
+    c.M = (long)op->M;
+    c.Q = (long)op->Q;
+    c.nElmt = op->nElmt;
+    return imf::dense_pays(c);
 }
 
 // The element matrices of a collapsed-shape operator for the dense kernel, read off the
@@ -357,7 +349,7 @@ bool dense_pays(const imf_op op, int tr, bool helm, bool from_modes)
 // chosen so that one metric term remains: rows e_a give K_aa; a single row e_a + e_b or
 // e_a - e_b gives K_aa + K_bb + (K_ab + K_ba) or the same with a minus sign.
 // Taken by BwdTrans, IProduct and their transposes and by Helmholtz with one set of factors
-// per element and at most 128 modes, where dense_pays().
+// per element and at most 128 modes, where dense_pays() (mf_routes.hpp).
 int build_dense(imf_op op)
 {
     const int M = (int)op->M, Q = (int)op->Q;

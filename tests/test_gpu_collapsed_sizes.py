@@ -105,3 +105,48 @@ def test_dbdata_that_is_not_d_bdata_is_still_used(shape):
         o.set_lambda(0.0)
         got.append(o.apply(u).cpu().numpy())
     assert _rel(got[1], 2.0 * got[0]) < 1e-12
+
+
+@pytest.mark.parametrize("shape,kind,deformed,nm,extra,E", [
+    ("tri", "BwdTrans", False, 5, 1, 6001), ("tet", "Helmholtz", False, 6, 1, 3743),
+    ("tet", "Helmholtz", False, 8, 4, 319), ("tet", "IProduct", False, 5, 1, 4561),
+    ("tet", "IProduct", True, 5, 1, 7745), ("pyr", "IProduct", False, 3, 1, 3507),
+    ("prism", "IProduct", False, 2, 1, 3009), ("tet", "BwdTrans", False, 3, 1, 30005),
+    ("tet", "BwdTrans", False, 5, 4, 1231), ("prism", "BwdTrans", False, 5, 8, 607),
+    ("pyr", "IProduct", True, 4, 4, 5951), ("prism", "Helmholtz", False, 4, 1, 12811),
+    ("tet", "IProduct", False, 8, 4, 3509)])
+def test_large_element_counts_agree_with_small_ones(shape, kind, deformed, nm, extra, E):
+    """Element counts just beyond those from which an operator takes dense products, with a ragged
+    last tile: the first, some middle and the last elements equal those of an operator of 65
+    elements, whose kernel is another one (checked against the oracle above).  Both directions
+    (the transpose of one direction of a transform is the other's kernel)."""
+    print(f"[case] {shape} {kind} nm={nm} nq=+{extra} E={E} deformed={deformed}", flush=True)
+    nq = nm + extra
+    rng = np.random.default_rng(E)
+    R = np.array(REG[shape], dtype=float)
+    jitter = 0.1 if deformed or shape in ("tri", "tet") else 0.0
+    verts = R[None] * rng.uniform(0.5, 2.0, (E, 1, 1)) + jitter * rng.uniform(-1, 1, (E,) + R.shape)
+    b = _basis(shape, nm, nq)
+    nqs = tuple(b[f"nq{d}"] for d in range(R.shape[1]))
+    geo = "Deformed" if deformed else "Regular"
+
+    def op(v):
+        n = len(v)
+        o = H.Operator(f"{kind}_{shape.capitalize()}_{geo}", nm, nqs, n, basis=_tables(shape, b))
+        jac, df = H.geom_device(shape, torch.from_numpy(v).cuda(), nqs, None, deformed)
+        if o.needs_jac():
+            o.set_jac(jac)
+        if o.needs_df():
+            o.set_df(df)
+            o.set_lambda(2.5)
+        return o
+    big = op(verts)
+    sizes = {"Helmholtz": (b["M"], b["M"]), "BwdTrans": (b["M"], b["Q"]), "IProduct": (b["Q"], b["M"])}[kind]
+    for transpose in (False, True) if kind != "Helmholtz" else (False,):
+        ni, no = sizes[::-1] if transpose else sizes
+        x = torch.from_numpy(rng.uniform(-1, 1, (E, ni))).cuda()
+        run = lambda o, v: (o.apply_transpose if transpose else o.apply)(v.reshape(-1).contiguous())
+        y = run(big, x).reshape(E, no)
+        for a in (0, E // 2, E - 65):
+            part = run(op(verts[a:a + 65].copy()), x[a:a + 65]).reshape(65, no)
+            assert _rel(y[a:a + 65].cpu().numpy(), part.cpu().numpy()) < 1e-12, (transpose, a)
