@@ -418,33 +418,15 @@ constexpr int helm_geo_prefetch()
     return per > 56 ? 0 : (56 / per > 7 ? 7 : 56 / per);
 }
 
-// Whether a launch packs elements into 256-thread workgroups (HexCfg).  Measured at 12e6
-// points, nq - 1 modes, narrow / wide in us: 6 points FP64 regular 98/74, deformed 152/137;
-// 9 points 123/110, 205/183; 7 points FP32 regular 57/50, but FP64 133/150 deformed; 6 points
-// FP32 regular 64/47, deformed 74/79; 5 points FP64 70/70, 121/127.  BwdTrans, IProduct and
-// PhysDeriv, bound by HBM, gain nothing (7 points: IProduct 51/70, PhysDeriv 76/101).
-template <int NQ, typename T, int GEO, bool MANY>
-constexpr bool helm_wide()
-{
-    if (MANY) return false;  // the geometry staged in LDS takes the room
-    constexpr bool f64 = sizeof(T) == 8;
-    if (NQ == 6) return f64 || GEO != kDeformed;
-    if (NQ == 7) return !f64 && GEO != kDeformed;
-    return NQ == 9;
-}
-
-template <int NQ, typename T, int GEO, bool MANY>
-using HelmCfg = HexCfg<NQ, helm_wide<NQ, T, GEO, MANY>()>;
-
-template <int NM, int NQ, typename T, int GEO, bool GATHER = false, bool MANY = false>
-__global__ __launch_bounds__((HelmCfg<NQ, T, GEO, MANY>::BLOCK)) void hex_helmholtz_kernel(
+template <int NM, int NQ, typename T, int GEO, bool WIDE = false, bool GATHER = false, bool MANY = false>
+__global__ __launch_bounds__((HexCfg<NQ, WIDE>::BLOCK)) void hex_helmholtz_kernel(
     const Tab<NM, NQ, T> tab, int nElmt, T lambda, const T *__restrict__ in,
     const T *__restrict__ geom, T *__restrict__ out, const int *__restrict__ gmap = nullptr,
     const signed char *__restrict__ gsign = nullptr, int nvec = 1, long ldin = 0,
     long ldout = 0, const int *__restrict__ skip = nullptr)
 {
     if (GATHER && skip && *skip) return;
-    using C = HelmCfg<NQ, T, GEO, MANY>;
+    using C = HexCfg<NQ, WIDE>;
     using Lb = HexLds<NM, NQ>;
     constexpr int M = Lb::M, Q = Lb::Q, TPE = C::TPE;
     constexpr long GS = geo_stride(7 * Q, sizeof(T));

@@ -11,6 +11,7 @@
 #include "imf_common.hpp"
 #include "mf_hex_kernels.hpp"
 #include "mf_quad_kernels.hpp"
+#include "mf_routes.hpp"
 
 namespace imf {
 
@@ -26,24 +27,34 @@ hipError_t launch_hex(const LaunchArgs &a)
     const T *geom = static_cast<const T *>(a.geom);
     T *out = static_cast<T *>(a.out);
     if constexpr (KIND == kHelmholtz) {
-        using W = HelmCfg<NQ, T, GEO, false>;
-        const dim3 wgrid((unsigned)((a.nElmt + W::EPB - 1) / W::EPB)), wblock(W::BLOCK);
-        if constexpr (std::is_same_v<T, double>) {
-            if (a.gmap) {
-                hex_helmholtz_kernel<NM, NQ, T, GEO, true><<<wgrid, wblock, 0, a.stream>>>(
-                    tab, a.nElmt, T(a.lambda), in, geom, out, a.gmap, a.gsign, 1, 0, 0, a.skip);
-                return hipGetLastError();
-            }
-        }
-        if (a.gmap) return hipErrorInvalidValue;  // gathered input: FP64 only
-        if (a.nvec > 1) {
-            hex_helmholtz_kernel<NM, NQ, T, GEO, false, true><<<grid, block, 0, a.stream>>>(
+        if (!a.gmap && a.nvec > 1) {  // narrow: the geometry staged in LDS takes the room
+            hex_helmholtz_kernel<NM, NQ, T, GEO, false, false, true><<<grid, block, 0, a.stream>>>(
                 tab, a.nElmt, T(a.lambda), in, geom, out, nullptr, nullptr, a.nvec, a.ldin,
                 a.ldout);
             return hipGetLastError();
         }
-        hex_helmholtz_kernel<NM, NQ, T, GEO>
-            <<<wgrid, wblock, 0, a.stream>>>(tab, a.nElmt, T(a.lambda), in, geom, out);
+        auto launch = [&](auto wide) {
+            constexpr bool WIDE = decltype(wide)::value;
+            using W = HexCfg<NQ, WIDE>;
+            const dim3 g((unsigned)((a.nElmt + W::EPB - 1) / W::EPB)), b(W::BLOCK);
+            if constexpr (std::is_same_v<T, double>) {
+                if (a.gmap) {
+                    hex_helmholtz_kernel<NM, NQ, T, GEO, WIDE, true><<<g, b, 0, a.stream>>>(
+                        tab, a.nElmt, T(a.lambda), in, geom, out, a.gmap, a.gsign, 1, 0, 0, a.skip);
+                    return;
+                }
+            }
+            hex_helmholtz_kernel<NM, NQ, T, GEO, WIDE>
+                <<<g, b, 0, a.stream>>>(tab, a.nElmt, T(a.lambda), in, geom, out);
+        };
+        if (a.gmap && !std::is_same_v<T, double>) return hipErrorInvalidValue;  // gathered input: FP64 only
+        if constexpr (constexpr int from = helm_wide_from(NQ, std::is_same_v<T, double>, GEO == kDeformed); from > 0) {
+            if (a.nElmt >= from) {
+                launch(std::true_type{});
+                return hipGetLastError();
+            }
+        }
+        launch(std::false_type{});
     } else if constexpr (KIND == kMass) {
         hex_mass_kernel<NM, NQ, T, GEO><<<grid, block, 0, a.stream>>>(
             tab, a.nElmt, a.nvec, in, a.ldin, geom, out, a.ldout);

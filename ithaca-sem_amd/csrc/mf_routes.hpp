@@ -1,9 +1,28 @@
-// When a collapsed-shape operator takes dense products over its elements (mf_dense.hip).
-// Plain C++, so that the rule can be checked without a device.
+// Which kernel or launch shape an operator takes by its sizes: rules that weigh two measured
+// alternatives.  Plain C++, so that they can be checked without a device.
 #pragma once
 
 namespace imf {
 
+// Hex Helmholtz: the number of elements from which a launch packs them into 256-thread workgroups (HexCfg); 0:
+// never.  Many elements fill the lanes that an element of its own workgroup leaves idle, few are
+// spread over more CUs and wait for no other element's barriers.  Narrow / wide in us, nq - 1 modes:
+//   6 points FP64 deformed   16: 5.9/7.6   1 000: 8.0/8.8    4 000: 15.6/15.8   50 000: 131/118
+//            FP64 regular    16: 5.6/6.7   1 000: 6.5/7.3    4 000: 11.3/10.9   50 000: 84/64
+//   9 points FP64 deformed   16: 10.6/13.0 1 000: 17.9/18.9  1 500: 28.8/20.4   50 000: 585/536
+//            FP32 deformed   16: 7.2/8.4   1 000: 12.0/12.9  1 500: 15.7/14.3   50 000: 265/237
+//   7 points FP32 regular    16: 5.9/6.8   4 000: 10.8/11.2  8 000: 16.3/15.7   50 000: 74/69
+// Never ahead at 12e6 points: 7 points FP64 deformed 133/150, 6 points FP32 deformed 74/79,
+// 5 points FP64 70/70 and 121/127; BwdTrans, IProduct and PhysDeriv are bound by HBM (7 points:
+// IProduct 51/70, PhysDeriv 76/101).
+constexpr int helm_wide_from(int nq, bool f64, bool deformed)
+{
+    if (nq == 6) return f64 || !deformed ? 4000 : 0;
+    if (nq == 7) return !f64 && !deformed ? 8000 : 0;
+    return nq == 9 ? 1500 : 0;
+}
+
+// When a collapsed-shape operator takes dense products over its elements (mf_dense.hip).
 struct DenseCase {
     int shape;            // kRouteTri ...
     bool helm;            // Helmholtz; else a transform

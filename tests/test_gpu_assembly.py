@@ -462,3 +462,19 @@ def test_iteration_limit_at_and_around_convergence(nm, nq, lam):
     # the preconditioner's diagonal: with it the solve takes no more iterations than the bound of
     # a Jacobi-scaled system of this size (a wrong diagonal takes several times more)
     assert it < 60 * nm
+
+
+def test_helmsolve_of_many_hexes_satisfies_the_operator():
+    """4 096 elements of 4 modes and 6 points, beyond the count from which the gathered Helmholtz
+    kernel packs elements into 256 threads: the plain operator on the solution gives the right-hand
+    side back on the free modes (bar: twice the solver's own relative residual, whose norm this is)."""
+    verts, ids = _mesh(16, True, seed=8, jitter=0.02)
+    print("[case] helmsolve 16^3 nm=4 nq=6", flush=True)
+    A, Hop, rhs, _ = _gpu_problem(verts, ids, 4, 6, 10.0)
+    x, it, res = A.helmsolve(Hop, rhs, tol=1e-9)
+    _, _, bnd, _ = assembly.assembly_map_hex(ids, 4)
+    free = torch.ones(A.nglobal, dtype=torch.bool, device="cuda")
+    l2g = assembly.assembly_map_hex(ids, 4)[0]
+    free[torch.from_numpy(l2g[bnd.astype(bool)].astype(np.int64)).cuda()] = False
+    r = (rhs - A.assemble(Hop.apply(A.global_to_local(x))))[free]
+    assert res <= 1e-9 and float(r.norm()) <= 2e-9 * float(rhs.norm())

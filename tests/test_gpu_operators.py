@@ -445,3 +445,27 @@ def test_helmholtz_and_mass_tables(shape, nm, nq, E):
         if dim == 3:
             m = O.iproduct("hex", b, E, deformed, jac, O.bwdtrans("hex", b, E, u))
             assert rel(_op(f"Mass_{geo}", nm, nq, E, b, jac).apply(_dev(u)).cpu().numpy(), m) < TOL64
+
+
+@pytest.mark.parametrize("nm,nq,E,prec", [(5, 6, 4003, "fp64"), (4, 6, 4003, "fp32"), (7, 9, 1501, "fp64"),
+                                          (8, 9, 1502, "fp32"), (5, 7, 8004, "fp32")])
+@pytest.mark.parametrize("deformed", [False, True])
+def test_helmholtz_of_many_hexes_agrees_with_few(nm, nq, E, prec, deformed):
+    """Element counts just beyond those from which elements are packed into 256 threads, with a
+    ragged last workgroup: the first, middle and last elements equal those of an operator of 65."""
+    print(f"[case] nm={nm} nq={nq} E={E} {prec} deformed={deformed}", flush=True)
+    rng = np.random.default_rng(E)
+    v = mesh.hex_box(1, 0.0, rng) * rng.uniform(0.5, 2.0, (E, 1, 1))
+    v = v + (0.1 * rng.uniform(-1, 1, v.shape) if deformed else 0.0)
+    b = O.basis(nm, nq)
+    p = H.FP64 if prec == "fp64" else H.FP32
+    u = torch.from_numpy(rng.uniform(-1, 1, (E, nm ** 3))).cuda().to(torch.float64 if p == H.FP64 else torch.float32)
+
+    def run(a, n):
+        jac, df = H.geom_device("hex", torch.from_numpy(v[a:a + n].copy()).cuda(), nq, b["z"], deformed)
+        op = _op(f"Helmholtz_Hex_{'Deformed' if deformed else 'Regular'}", nm, nq, n, b, jac, df, prec=p)
+        op.set_lambda(2.5)
+        return op.apply(u[a:a + n].reshape(-1).contiguous()).reshape(n, -1).double().cpu().numpy()
+    y = run(0, E)
+    for a in (0, E // 2, E - 65):
+        assert rel(y[a:a + 65], run(a, 65)) < (1e-13 if p == H.FP64 else TOL32)

@@ -1,6 +1,7 @@
-"""The rule that gives a collapsed-shape operator to the dense-product kernel, compiled from its
-header and asked about measured points: (shape, dense time, time of the kernel it replaces) at an
-element count.  Where the two are 1.5 times apart or more, the rule takes the faster one."""
+"""The rules that choose a kernel or a launch shape by size, compiled from their header and asked
+about measured points: the dense-product kernel of the collapsed shapes against the kernel it
+replaces (1.5 times apart or more), and the wide launch of the hex Helmholtz kernels.  The rule
+takes the faster one."""
 import math
 import os
 import subprocess
@@ -14,7 +15,10 @@ MAIN = """
 int main() {
     int s, h, f, p, c; long M, Q, n;
     while (std::scanf("%d %d %d %d %d %ld %ld %ld", &s, &h, &f, &p, &c, &M, &Q, &n) == 8)
-        std::printf("%d\\n", imf::dense_pays({s, h != 0, f != 0, p != 0, c != 0, M, Q, n}));
+        if (s < 0)  // hex Helmholtz: points, FP64, deformed, elements
+            std::printf("%d\\n", imf::helm_wide_from(h, f, p) > 0 && n >= imf::helm_wide_from(h, f, p));
+        else
+            std::printf("%d\\n", imf::dense_pays({s, h != 0, f != 0, p != 0, c != 0, M, Q, n}));
 }
 """
 SHAPES = ["tri", "tet", "prism", "pyr"]
@@ -90,3 +94,13 @@ def test_the_choice_changes_once_with_the_number_of_elements(ask):
     for i, k in enumerate(keys):
         one = got[i * len(ns):(i + 1) * len(ns)]
         assert one == sorted(one), k
+
+
+@pytest.mark.parametrize("nq,fp64,deformed,n,narrow,wide", [
+    (6, 1, 1, 16, 5.9, 7.6), (6, 1, 1, 1000, 8.0, 8.8), (6, 1, 1, 6000, 22.1, 20.1), (6, 1, 0, 400, 6.0, 7.1),
+    (6, 1, 0, 6000, 14.5, 12.8), (6, 0, 0, 2000, 6.7, 7.3), (6, 0, 0, 6000, 10.9, 9.9), (9, 1, 1, 256, 11.5, 13.6),
+    (9, 1, 1, 1500, 28.8, 20.4), (9, 0, 0, 1000, 9.2, 10.1), (9, 0, 0, 1500, 12.5, 10.5), (9, 0, 1, 100, 7.5, 9.2),
+    (9, 0, 1, 3000, 23.6, 21.7), (7, 0, 0, 3000, 9.3, 9.8), (7, 0, 0, 16000, 26.6, 24.4), (7, 1, 1, 35000, 133, 150),
+    (6, 0, 1, 55000, 74, 79)])
+def test_hex_helmholtz_launch(ask, nq, fp64, deformed, n, narrow, wide):
+    assert ask([(-1, nq, fp64, deformed, 0, 0, 0, n)]) == [wide < narrow]
