@@ -128,7 +128,7 @@ struct LaunchArgs {
     // mode as gsign[i] * in[gmap[i]] (GlobalToLocal fused into the operator's load)
     const int *gmap = nullptr;
     const signed char *gsign = nullptr;
-    const int *skip = nullptr;  // with gmap: the kernel returns when *skip is non-zero
+    const int *skip = nullptr;  // Helmholtz: the kernel returns when *skip is non-zero
 };
 using LaunchFn = hipError_t (*)(const LaunchArgs &);
 

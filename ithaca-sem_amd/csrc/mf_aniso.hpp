@@ -21,6 +21,7 @@ struct AnisoArgs {
     const double *df;   // GetDerivFactors layout: [9][nElmt*Q] deformed, [9][nElmt] regular
     int nvec = 1;
     long ldin = 0, ldout = 0;
+    const int *skip = nullptr;  // the kernel returns when *skip is non-zero
 };
 
 __host__ __device__ inline int aniso_table_len(const int *nm, const int *nq)

@@ -364,8 +364,10 @@ int build_map(int shape, int E, const int *nm, bool per_dir, const long long *vi
 // --------------------------------------------------------------------------- kernels
 // local = sign * global[l2g]   (Vmath::Gathr with signs)
 __global__ void g2l_kernel(long n, const int *__restrict__ l2g, const signed char *__restrict__ sg,
-                           const double *__restrict__ glob, double *__restrict__ loc)
+                           const int *__restrict__ skip, const double *__restrict__ glob,
+                           double *__restrict__ loc)
 {
+    if (skip && *skip) return;
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) loc[i] = sg[i] * glob[l2g[i]];
 }
@@ -398,12 +400,6 @@ __global__ void assemble_kernel(long ng, const int *__restrict__ off, const unsi
 {
     const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (g < ng) glob[g] = assemble_one<kUnsigned>(g, off, inv, loc, mask);
-}
-
-__global__ void zero_kernel(long n, double *__restrict__ x)
-{
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) x[i] = 0.0;
 }
 
 struct DiagTab {
@@ -513,7 +509,7 @@ __global__ void inv_masked(long n, const unsigned char *__restrict__ mask, doubl
 // Scalars of the conjugate-gradient iteration, kept on the device so that the next kernels
 // can be queued without waiting for them.
 struct CgState {
-    double rho, mu, eps, alpha, beta, thr, rhs_mag;
+    double rho, eps, alpha, beta, thr, rhs_mag;
     int it;    // iterations as the reference counts them
     int done;  // the tolerance is reached: the kernels of later iterations return at once
 };
@@ -529,11 +525,15 @@ __global__ void cg_init(long n, const unsigned char *__restrict__ mask, const do
 }
 
 // w = dinv * r
-__global__ void cg_precon(long n, const double *__restrict__ dinv, const double *__restrict__ r,
-                          double *__restrict__ w)
+__global__ void cg_precon(long n, const CgState *__restrict__ st, const double *__restrict__ dinv,
+                          const double *__restrict__ r, double *__restrict__ w,
+                          double *__restrict__ p, double *__restrict__ q)
 {
+    if (st->done) return;
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) w[i] = dinv[i] * r[i];
+    if (i >= n) return;
+    w[i] = dinv[i] * r[i];
+    p[i] = q[i] = 0.0;
 }
 
 // p = w + beta p; q = s + beta q; x += alpha p; r -= alpha q; w = dinv r
@@ -702,9 +702,10 @@ inline unsigned nblk(long n) { return (unsigned)((n + RB - 1) / RB); }
 
 // y = R x for the Robin matrix R in CSR form over the global modes
 __global__ void csr_spmv(long ng, const int *__restrict__ off, const int *__restrict__ col,
-                         const double *__restrict__ val, const double *__restrict__ x,
-                         double *__restrict__ y)
+                         const double *__restrict__ val, const int *__restrict__ skip,
+                         const double *__restrict__ x, double *__restrict__ y)
 {
+    if (*skip) return;
     const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= ng) return;
     double s = 0.0;
@@ -769,27 +770,22 @@ int apply_global_dots(imf_asm a, int nops, const imf_op *ops, const double *w, c
                       double *out, bool first, hipStream_t s)
 {
     double *l0 = a->d_loc, *l1 = a->d_loc + a->nloc;
-    const bool any_aniso = std::any_of(ops, ops + nops, [](const imf_op o) { return o->aniso; });
-    if (a->shape == imf::kHex && !any_aniso) {  // GlobalToLocal fused into the coefficient load
-        long e0 = 0;
-        for (int g = 0; g < nops; ++g) {
-            const long o = a->loff[e0];
-            if (int st = imf_apply_gather_device(ops[g], w, a->d_l2g + o, a->d_sg + o, l1 + o,
-                                                 &a->d_state->done, s))
-                return st;
-            e0 += ops[g]->nElmt;
-        }
-    } else {
-        g2l_kernel<<<nblk(a->nloc), RB, 0, s>>>(a->nloc, a->d_l2g, a->d_sg, w, l0);
-        long e0 = 0;
-        for (int g = 0; g < nops; ++g) {
-            const long o = a->loff[e0];
-            if (int st = imf_apply_device(ops[g], l0 + o, l1 + o, s)) return st;
-            e0 += ops[g]->nElmt;
-        }
+    const int *skip = &a->d_state->done;
+    // isotropic hexes gather their coefficients themselves (GlobalToLocal fused into the load)
+    auto gathers = [&](const imf_op o) { return a->shape == imf::kHex && !o->aniso; };
+    if (!std::all_of(ops, ops + nops, gathers))
+        g2l_kernel<<<nblk(a->nloc), RB, 0, s>>>(a->nloc, a->d_l2g, a->d_sg, skip, w, l0);
+    long e0 = 0;
+    for (int g = 0; g < nops; ++g) {
+        const long o = a->loff[e0];
+        const bool own = gathers(ops[g]);
+        if (int st = imf_apply_skip_device(ops[g], own ? w : l0 + o, own ? a->d_l2g + o : nullptr,
+                                           own ? a->d_sg + o : nullptr, l1 + o, skip, s))
+            return st;
+        e0 += ops[g]->nElmt;
     }
     if (a->r_nnz)
-        csr_spmv<<<nblk(a->ng), RB, 0, s>>>(a->ng, a->d_roff, a->d_rcol, a->d_rval, w, a->d_rw);
+        csr_spmv<<<nblk(a->ng), RB, 0, s>>>(a->ng, a->d_roff, a->d_rcol, a->d_rval, skip, w, a->d_rw);
     const int nb = (int)std::min<long>(kAsmParts, nblk(a->ng));
     assemble_dot3_kernel<<<nb, RB, 0, s>>>(a->ng, a->d_off, a->d_inv, l1, a->d_mask,
                                            a->r_nnz ? a->d_rw : nullptr, a->d_state, r, w, out,
@@ -1039,7 +1035,8 @@ int imf_assembly_set_robin(imf_asm a, long nnz, const int *rows, const int *cols
 int imf_global_to_local_device(imf_asm a, const double *d_global, double *d_local, void *stream)
 {
     if (!a || !d_global || !d_local) return afail(IMF_ERR_ARG, "imf_global_to_local_device: null argument");
-    g2l_kernel<<<nblk(a->nloc), RB, 0, (hipStream_t)stream>>>(a->nloc, a->d_l2g, a->d_sg, d_global, d_local);
+    g2l_kernel<<<nblk(a->nloc), RB, 0, (hipStream_t)stream>>>(a->nloc, a->d_l2g, a->d_sg, nullptr,
+                                                             d_global, d_local);
     ACHECK(hipGetLastError(), "g2l_kernel");
     return IMF_OK;
 }
@@ -1142,38 +1139,45 @@ int imf_helmsolve_cg_groups_device(imf_asm a, int nops, const imf_op *ops, const
         dot3_partial<<<a->nparts, RB, 0, s>>>(ng, x0, x1, x2, a->d_part);
     };
     // rhs magnitude over all global modes (Set_Rhs_Magnitude), the first residual and the first
-    // direction; then iterations in groups of four, a copy of the scalars after each.  The host
-    // waits for the scalars of the group before the one it has just queued, so the device always
-    // has work; iterations queued past the last one return at once.
+    // direction; then iterations in groups of one, two and from then on four, a copy of the scalars
+    // after each.  The host waits for the scalars of the group before the one it has just queued,
+    // so the device always has work; the kernels of iterations queued past the last one return at
+    // once, and none are queued when the first residual is small enough.
+    auto post = [&](int b) -> int {
+        ACHECK(hipMemcpyAsync(a->h_state + b, a->d_state, sizeof(CgState), hipMemcpyDeviceToHost, s), "copy");
+        ACHECK(hipEventRecord(a->ev[b], s), "event");
+        return IMF_OK;
+    };
     dots(d_rhs, d_rhs, d_rhs);
     cg_scalars<0><<<1, FB, 0, s>>>(a->nparts, a->d_part, tol, a->d_state);
     cg_init<<<nblk(ng), RB, 0, s>>>(ng, a->d_mask, d_rhs, r, d_x);
     dots(r, r, r);
     cg_scalars<1><<<1, FB, 0, s>>>(a->nparts, a->d_part, tol, a->d_state);
-    cg_precon<<<nblk(ng), RB, 0, s>>>(ng, dinv, r, w);
-    zero_kernel<<<nblk(2 * ng), RB, 0, s>>>(2 * ng, p);  // p and q
+    if (int st = post(0)) return st;
+    cg_precon<<<nblk(ng), RB, 0, s>>>(ng, a->d_state, dinv, r, w, p, q);
     ACHECK(hipGetLastError(), "cg set-up kernels");
     if (int st = apply_global_dots(a, nops, ops, w, r, sv, true, s)) return st;
-    constexpr int kGroup = 4;
-    CgState last{};
-    long queued = 0;
-    for (int b = 0, first = 1;; b ^= 1, first = 0) {
-        const long upto = std::min<long>(std::max(max_iter, 0), queued + kGroup);
-        for (; queued < upto; ++queued) {
+    ACHECK(hipEventSynchronize(a->ev[0]), "sync");
+    CgState last = a->h_state[0];
+    long queued = 0, group = 1;
+    for (int b = 1, before = 0; !last.done; b ^= 1, before = 1, group = std::min<long>(2 * group, 4)) {
+        if (queued >= max_iter) {
+            if (before) {
+                ACHECK(hipEventSynchronize(a->ev[b ^ 1]), "sync");
+                last = a->h_state[b ^ 1];
+            } else {
+                last.it = 1;  // the first direction
+            }
+            break;
+        }
+        for (const long upto = std::min<long>(max_iter, queued + group); queued < upto; ++queued) {
             cg_update<<<nblk(ng), RB, 0, s>>>(ng, a->d_state, dinv, p, q, w, sv, d_x, r);
             if (int st = apply_global_dots(a, nops, ops, w, r, sv, false, s)) return st;
         }
-        ACHECK(hipMemcpyAsync(a->h_state + b, a->d_state, sizeof(CgState), hipMemcpyDeviceToHost, s), "copy");
-        ACHECK(hipEventRecord(a->ev[b], s), "event");
-        if (!first) {
+        if (int st = post(b)) return st;
+        if (before) {
             ACHECK(hipEventSynchronize(a->ev[b ^ 1]), "sync");
             last = a->h_state[b ^ 1];
-            if (last.done) break;
-        }
-        if (queued >= max_iter) {
-            ACHECK(hipEventSynchronize(a->ev[b]), "sync");
-            last = a->h_state[b];
-            break;
         }
     }
     ACHECK(hipStreamSynchronize(s), "sync");

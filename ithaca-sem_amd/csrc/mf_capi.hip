@@ -437,8 +437,9 @@ int run(imf_op op, imf::LaunchFn fn, const void *in, void *out, void *stream, in
     }
     if (op->aniso) {
         if (gmap) return fail(IMF_ERR_UNSUPPORTED, "gathered input: isotropic operators only");
-        hipError_t e = imf::launch_aniso(aniso_args(op, in, out, nvec, ldin, ldout),
-                                         (hipStream_t)stream);
+        imf::AnisoArgs a = aniso_args(op, in, out, nvec, ldin, ldout);
+        a.skip = skip;
+        hipError_t e = imf::launch_aniso(a, (hipStream_t)stream);
         if (e != hipSuccess) return hip_fail(e, "kernel launch");
         return IMF_OK;
     }
@@ -916,15 +917,17 @@ imf::AnisoArgs aniso_args(const imf_op_s *op, const void *in, void *out, int nve
     return a;
 }
 
-int imf_apply_gather_device(imf_op_s *op, const double *glob, const int *gmap,
-                            const signed char *gsign, double *out, const int *skip,
-                            hipStream_t stream)
+int imf_apply_skip_device(imf_op_s *op, const double *in, const int *gmap,
+                          const signed char *gsign, double *out, const int *skip,
+                          hipStream_t stream)
 {
     if (int s = check_op(op)) return s;
-    if (op->kind != imf::kHelmholtz || op->shape != imf::kHex || op->prec != IMF_FP64 ||
-        op->aniso || !gmap || !gsign)
-        return fail(IMF_ERR_UNSUPPORTED, "gathered input: FP64 Helmholtz_Hex only");
-    return run(op, op->fwd, glob, out, stream, 1, 0, 0, gmap, gsign, skip);
+    const bool gathers = op->shape == imf::kHex && !op->aniso;
+    if (op->kind != imf::kHelmholtz || op->collapsed || op->prec != IMF_FP64 ||
+        gathers != (gmap && gsign))
+        return fail(IMF_ERR_UNSUPPORTED, "solver's apply: FP64 Helmholtz, gathered input for "
+                                         "isotropic hexes only");
+    return run(op, op->fwd, in, out, stream, 1, 0, 0, gmap, gsign, skip);
 }
 
 extern "C" {

@@ -83,6 +83,7 @@ __device__ void iprod(const Sizes &z, const double *f, double *a, double *b, Sto
 
 __global__ __launch_bounds__(256) void hex_aniso_kernel(AnisoArgs g)
 {
+    if (g.skip && *g.skip) return;
     extern __shared__ double sm[];
     Sizes z;
     for (int d = 0; d < 3; ++d) {

@@ -84,7 +84,7 @@ hipError_t launch_quad(const LaunchArgs &a)
     T *out = static_cast<T *>(a.out);
     if constexpr (KIND == kHelmholtz) {
         quad_helmholtz_kernel<NM, NQ, T, GEO>
-            <<<grid, block, 0, a.stream>>>(tab, a.nElmt, T(a.lambda), in, geom, out);
+            <<<grid, block, 0, a.stream>>>(tab, a.nElmt, T(a.lambda), in, geom, out, a.skip);
     } else if constexpr (KIND == kIProdDeriv) {
         quad_iprod_deriv_kernel<NM, NQ, T, GEO>
             <<<grid, block, 0, a.stream>>>(tab, a.nElmt, in, geom, out);

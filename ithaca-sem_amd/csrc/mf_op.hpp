@@ -62,10 +62,10 @@ struct imf_op_s {
 imf::AnisoArgs aniso_args(const imf_op_s *op, const void *in, void *out, int nvec, long ldin,
                           long ldout);
 
-// FP64 hex Helmholtz with its input gathered from a global vector: out = H(local), where
-// local[i] = gsign[i] * glob[gmap[i]] (GlobalToLocal fused into the kernel's load).
-// skip (device, may be null): nothing is done when it holds a non-zero value at the time the
-// kernel runs.  Library-internal (used by the assembled solver); defined in mf_capi.hip.
-int imf_apply_gather_device(imf_op_s *op, const double *glob, const int *gmap,
-                            const signed char *gsign, double *out, const int *skip,
-                            hipStream_t stream);
+// FP64 Helmholtz on quads and hexes that does nothing when *skip (device) is non-zero at the time
+// the kernel runs.  Isotropic hexes, and they alone, take a map: their input is gathered from a
+// global vector, out = H(local) with local[i] = gsign[i] * in[gmap[i]] (GlobalToLocal fused into
+// the kernel's load).  Library-internal (used by the assembled solver); defined in mf_capi.hip.
+int imf_apply_skip_device(imf_op_s *op, const double *in, const int *gmap,
+                          const signed char *gsign, double *out, const int *skip,
+                          hipStream_t stream);

@@ -159,13 +159,15 @@ __global__ __launch_bounds__(QuadCfg<NQ>::BLOCK) void quad_iproduct_kernel(
     quad_lines_to_modes<NM, NQ, T, false>(tab, acc, out + e * M, valid, active, t, lds[es]);
 }
 
-// Packed geometry: deformed [e][4][Q] (Jw, JwG00, JwG01, JwG11); regular [e][4]
+// skip (may be null) points to a device flag that makes the kernel return (an iteration queued past
+// the solver's last).  Packed geometry: deformed [e][4][Q] (Jw, JwG00, JwG01, JwG11); regular [e][4]
 // (J, J G00, J G01, J G11) with the weights applied here.
 template <int NM, int NQ, typename T, int GEO>
 __global__ __launch_bounds__(QuadCfg<NQ>::BLOCK) void quad_helmholtz_kernel(
     const Tab<NM, NQ, T> tab, int nElmt, T lambda, const T *__restrict__ in,
-    const T *__restrict__ geom, T *__restrict__ out)
+    const T *__restrict__ geom, T *__restrict__ out, const int *__restrict__ skip)
 {
+    if (skip && *skip) return;
     using C = QuadCfg<NQ>;
     constexpr bool AGAIN = NQ >= 9;  // 6,8 deformed at 12e6 points: held 77 us, read again 80
     constexpr int M = NM * NM, Q = NQ * NQ;
