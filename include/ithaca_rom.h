@@ -93,10 +93,13 @@ int irom_batch_param_grad(irom_batch b, const double *d_A, const double *d_lambd
  *                    16-deep panel, FP64 across panels
  *   IROM_GRAM_BF16X3 hi/lo BF16 split, 3 BF16 MFMA products, FP32 accumulation within a
  *                    32-deep panel, FP64 across panels
+ * The split modes trade accuracy for the rate of large products.  Products of at most 64 vectors
+ * (m, n <= 64) are bound by reading X and Y; they are formed in FP64 in every mode.
  * X == Y (same pointer, m == n, ldx == ldy) computes only the upper blocks and mirrors;
  * so does a mode OR-ed with IROM_GRAM_SYMMETRIC_RESULT when m == n (the caller states
  * that X^T Y is symmetric, e.g. S^T (M S) with M symmetric).
- * d_work must hold irom_gram_workspace_size(m, n, K) bytes (split-K partial blocks). */
+ * d_work must hold irom_gram_workspace_size(m, n, K) bytes (split-K partial blocks); a smaller
+ * one is used as far as it goes, down to m n doubles for each 65 536 of K begun (at most 512). */
 enum irom_gram_mode { IROM_GRAM_FP64 = 0, IROM_GRAM_FP32X3 = 1, IROM_GRAM_BF16X3 = 2,
                       IROM_GRAM_SYMMETRIC_RESULT = 16 };
 size_t irom_gram_workspace_size(int m, int n, long K);

@@ -42,17 +42,20 @@ struct GramArgs {
     int nsplit;   // K slices
     int sym;      // only blocks bi <= bj (the caller's product is symmetric)
     int vec;      // X, Y rows 16-byte aligned: 16-byte loads
+    int spread;   // blocks follow one another over the XCDs (gram_block)
 };
 
 // Block id -> (K slice, C block).  Workgroups are dispatched to the 8 XCDs round-robin by
 // linear id, so ids L with the same L % 8 share an L2: every C block of one K slice is
 // given the same L % 8 and adjacent dispatch order, and the slice's X/Y panels are read
-// from HBM once per XCD instead of once per C block.
+// from HBM once per XCD instead of once per C block.  With fewer than eight slices that leaves
+// XCDs idle, so slices of more blocks than an XCD has CUs are spread over all of them (1500
+// vectors of 1 000 entries 809 -> 215 us; 300 of them, 25 blocks, 85 us here and 93 spread).
 __device__ __forceinline__ bool gram_block(const GramArgs &g, int &split, int &bi, int &bj)
 {
     const int L = blockIdx.x, xcd = L & 7, r = L >> 3;
-    split = 8 * (r / g.ntiles) + xcd;
-    int t = r % g.ntiles;
+    split = g.spread ? L / g.ntiles : 8 * (r / g.ntiles) + xcd;
+    int t = g.spread ? L % g.ntiles : r % g.ntiles;
     if (split >= g.nsplit) return false;
     if (!g.sym) {
         bi = t / g.nbj;
@@ -326,22 +329,24 @@ __global__ __launch_bounds__(64 * GramMode<MODE>::NW, GB == 64 ? 4 : 2) void gra
 }
 
 // C (row-major m x n, ldc) (+)= sum over splits of the partial blocks; for symmetric
-// products every entry below the diagonal is taken from its mirror above it (computed in
-// an upper or diagonal block), so the result is exactly symmetric.  A workgroup sums RO
-// outputs, RS threads each over every RS-th slice and then pairwise in LDS: with one thread
-// per output a 12 x 12 result read its 1024 slices one after another.
-constexpr int RO = 16, RS = 16;
-__global__ __launch_bounds__(RO * RS) void gram_reduce_kernel(
+// products every entry below the diagonal is its mirror above it (computed in an upper or
+// diagonal block), so the result is exactly symmetric.  A workgroup sums 256 / RS outputs, RS
+// threads each over every RS-th slice and then pairwise in LDS.  RS = 16 for many slices: with one
+// thread per output a 12 x 12 result read its 1024 slices one after another.  With few slices the
+// outputs alone fill the chip, and RS = 1 reads whole lines (4096 x 4096 of one slice, symmetric,
+// with its product of vectors of one entry: 563 us with RS = 16, now 106 us).
+template <int RS>
+__global__ __launch_bounds__(256) void gram_reduce_kernel(
     int m, int n, int nsplit, const double *__restrict__ part, double *__restrict__ C, long ldc,
     int accumulate, int symmetric)
 {
+    constexpr int RO = 256 / RS;
     __shared__ double sh[RS][RO];
     const int o = threadIdx.x % RO, q = threadIdx.x / RO;
     const long g = (long)blockIdx.x * RO + o, mn = (long)m * n;
-    const bool in = g < mn;
-    const int i = in ? (int)(g / n) : 0, j = in ? (int)(g - (long)i * n) : 0;
-    const bool mirror = symmetric && j < i;
-    const double *src = part + (mirror ? (long)j * n + i : (long)i * n + j);
+    const int i = g < mn ? (int)(g / n) : 0, j = g < mn ? (int)(g - (long)i * n) : 0;
+    const bool in = g < mn && !(symmetric && j < i);
+    const double *src = part + (long)i * n + j;
     double s = 0.0;
     if (in)
         for (int p = q; p < nsplit; p += RS) s += src[p * mn];
@@ -355,6 +360,10 @@ __global__ __launch_bounds__(RO * RS) void gram_reduce_kernel(
     if (q == 0 && in) {
         double *c = C + (long)i * ldc + j;
         *c = accumulate ? *c + sh[0][o] : sh[0][o];
+        if (symmetric && j > i) {
+            c = C + (long)j * ldc + i;
+            *c = accumulate ? *c + sh[0][o] : sh[0][o];
+        }
     }
 }
 
@@ -458,11 +467,16 @@ namespace {
 thread_local std::string g_gerr;
 
 // K slices of a product.  m, n <= 64: one slice per wave of at most 1024 workgroups, each at
-// least 512 deep.  Larger: a multiple of 8 (one K slice belongs to one XCD) such that the
-// workgroups fill whole rounds of those that are resident (two per CU, four with 64 x 64
-// blocks), at most four rounds, slices at least 512 deep.  With one slice per 65 536 of K,
-// 384 vectors of 1.7 million entries ran as 162 workgroups on 256 CUs: 10.3 ms, now 5.9 ms
-// (43 TFLOP/s of the upper triangle's entries).
+// least 512 deep.  Larger: as few as let the workgroups fill whole rounds of those that are
+// resident (two per CU, four with 64 x 64 blocks) to within a few per cent, a multiple of 8 from 8
+// on (one K slice belongs to one XCD), at most four rounds, slices at least 512 deep.  With one
+// slice per 65 536 of K, 384 vectors of 1.7 million entries ran as 162 workgroups on 256 CUs:
+// 10.3 ms, now 5.9 ms (43 TFLOP/s of the upper triangle's entries).  With 8 slices at least,
+// 4096 x 4096 products took eight times the workspace for nothing.
+// The kernel that keeps the whole of C in each wave's accumulators; its sums over the waves cost
+// 2 us where a few entries of 49 to 64 vectors are the whole product (K = 1: 13.4 against 11.4 us).
+bool skinny(int m, int n, long K) { return m <= 64 && n <= 64 && (K > 16 || (m <= 48 && n <= 48)); }
+
 long gram_skinny_wgs(long K) { return std::max<long>(1, std::min<long>(1024, K / 2048)); }
 
 long gram_blocks(int m, int n, bool sym, int gb)
@@ -474,9 +488,10 @@ long gram_blocks(int m, int n, bool sym, int gb)
 long gram_splits(long ntiles, long K, int gb)
 {
     const long most = std::max<long>(1, K / 512), res = gb == 64 ? 1024 : 512;
-    long best = std::min<long>(8, most);
+    const long first = std::min(most, std::min<long>(8, (res + ntiles - 1) / ntiles));
+    long best = first;
     double fill = 0.0;
-    for (long ns = 8; ns <= most && ns * ntiles <= 4 * res; ns += 8) {
+    for (long ns = first; ns <= most && ns * ntiles <= 4 * res; ns += ns < 8 ? 1 : 8) {
         const double f = double(ns * ntiles) / double(res * ((ns * ntiles + res - 1) / res));
         if (f > fill + 0.02) {
             fill = f;
@@ -543,7 +558,9 @@ int irom_gram(int mode, int m, int n, long K, const double *d_X, long ldx, const
     ga.Y = d_Y;
     ga.ldy = ldy;
     ga.part = (double *)d_work;
-    const int gb = base == IROM_GRAM_FP64 && gram_small_blocks(m, n, symmetric) ? 64 : 128;
+    // at most 64 vectors: bound by reading X and Y in every mode, so all take the FP64 products
+    const int prod = m <= 64 && n <= 64 ? (int)IROM_GRAM_FP64 : base;
+    const int gb = prod == IROM_GRAM_FP64 && gram_small_blocks(m, n, symmetric) ? 64 : 128;
     ga.nbj = (n + gb - 1) / gb;
     ga.ntiles = (int)gram_blocks(m, n, symmetric, gb);
     ga.sym = symmetric;
@@ -555,8 +572,7 @@ int irom_gram(int mode, int m, int n, long K, const double *d_X, long ldx, const
     }
     double *part = (double *)d_work;
     const long fit = (long)(work_bytes / ((size_t)m * n * sizeof(double)));
-    if (m <= 64 && n <= 64) {
-        // bound by reading X and Y in every mode, so all modes take the FP64 products
+    if (skinny(m, n, K)) {
         const long nwg = std::min(gram_skinny_wgs(K), fit);
         ga.kchunk = ((K + 4 * nwg - 1) / (4 * nwg) + 15) / 16 * 16;
         ga.nsplit = (int)((K + 4 * ga.kchunk - 1) / (4 * ga.kchunk));
@@ -571,18 +587,22 @@ int irom_gram(int mode, int m, int n, long K, const double *d_X, long ldx, const
         const long nsplit = std::min(gram_splits(ga.ntiles, K, gb), fit);
         ga.kchunk = ((K + nsplit - 1) / nsplit + 31) / 32 * 32;
         ga.nsplit = (int)((K + ga.kchunk - 1) / ga.kchunk);
-        const unsigned grid = (unsigned)(8L * ga.ntiles * ((ga.nsplit + 7) / 8));
-        if (base == IROM_GRAM_FP64)
+        ga.spread = ga.nsplit < 8 && ga.ntiles > 32;
+        const unsigned grid = (unsigned)(ga.spread ? (long)ga.ntiles * ga.nsplit
+                                                   : 8L * ga.ntiles * ((ga.nsplit + 7) / 8));
+        if (prod == IROM_GRAM_FP64)
             (gb == 64 ? irom::gram_kernel<0, 64> : irom::gram_kernel<0, 128>)
                 <<<grid, 64 * irom::GramMode<0>::NW, 0, s>>>(ga);
-        else if (base == IROM_GRAM_FP32X3)
+        else if (prod == IROM_GRAM_FP32X3)
             irom::gram_kernel<1, 128><<<grid, 64 * irom::GramMode<1>::NW, 0, s>>>(ga);
         else
             irom::gram_kernel<2, 128><<<grid, 64 * irom::GramMode<2>::NW, 0, s>>>(ga);
     }
     const long tot = (long)m * n;
-    irom::gram_reduce_kernel<<<(unsigned)((tot + irom::RO - 1) / irom::RO), irom::RO * irom::RS, 0, s>>>(
-        m, n, ga.nsplit, part, d_C, ldc, accumulate, symmetric);
+    const int rs = ga.nsplit <= 8 ? 1 : ga.nsplit <= 32 && tot > 8192 ? 4 : 16;
+    (rs == 1 ? irom::gram_reduce_kernel<1> : rs == 4 ? irom::gram_reduce_kernel<4> : irom::gram_reduce_kernel<16>)
+        <<<(unsigned)((tot * rs + 255) / 256), 256, 0, s>>>(m, n, ga.nsplit, part, d_C, ldc, accumulate,
+                                                             symmetric);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         g_gerr = std::string("irom_gram: ") + hipGetErrorString(e);

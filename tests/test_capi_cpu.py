@@ -115,3 +115,16 @@ def test_create_rejects_bad_requests_without_gpu():
     st = lib.imf_create(b"Helmholtz_Hex_Deformed", 2, nm, nq, arr, arr, arr, arr, 8, 0,
                         ctypes.byref(h))
     assert st == 1
+
+
+def test_gram_workspace_of_large_products_is_a_few_results():
+    """Products whose blocks fill the chip with few slices of K ask for few partial results: 4 096
+    vectors at most four times m n doubles, where eight were asked for; one for a short K."""
+    from ithaca_hip import pod
+    L = pod._lib()
+    for m, K, most in ((4096, 4096, 4), (4096, 60000, 4), (3000, 10000, 5), (2048, 600, 1), (6000, 60000, 2)):
+        assert L.irom_gram_workspace_size(m, m, K) <= most * m * m * 8, (m, K)
+    # never less than irom_gram accepts
+    for m in (1, 12, 64, 65, 200, 2000):
+        for K in (1, 1000, 65537, 10 ** 7):
+            assert L.irom_gram_workspace_size(m, m, K) >= m * m * 8 * min(512, (K + 65535) // 65536)

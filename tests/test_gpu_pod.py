@@ -59,6 +59,54 @@ def test_gram_of_few_vectors(mode, m, n, K, pad):
     assert np.array_equal(gs, gs.T)
 
 
+@pytest.mark.parametrize("m,n,K", [(64, 64, 1), (49, 64, 16), (64, 50, 17), (300, 300, 900), (900, 1000, 700),
+                                   (1100, 1100, 2_100), (1300, 700, 5_200), (200, 260, 12_000)])
+def test_gram_of_few_slices(m, n, K):
+    """One to 32 slices of K: blocks spread over the chip or kept to an XCD, each form of the
+    reduction, with and without accumulation, symmetric (exactly) or not, whole and smallest
+    workspace.  Bar as above."""
+    print(f"[case] gram few slices m={m} n={n} K={K}", flush=True)
+    rng = np.random.default_rng(m + K)
+    X, Y, C0 = rng.standard_normal((m, K)), rng.standard_normal((n, K)), rng.standard_normal((m, n))
+    scale = np.linalg.norm(X, axis=1)[:, None] * np.linalg.norm(Y, axis=1)[None]
+    out = _dev(C0)
+    pod.gram(_dev(X), _dev(Y), out=out, accumulate=True)
+    assert (np.abs(out.cpu().numpy() - C0 - X @ Y.T) / (scale + np.abs(C0))).max() < 1e-13
+    if m == n:
+        got = pod.gram(_dev(X)).cpu().numpy()
+        nx = np.linalg.norm(X, axis=1)
+        assert np.array_equal(got, got.T)
+        assert (np.abs(got - X @ X.T) / (nx[:, None] * nx[None])).max() < 1e-13
+        out = _dev(C0)
+        pod.gram(_dev(X), out=out, accumulate=True)
+        assert (np.abs(out.cpu().numpy() - C0 - X @ X.T) / (nx[:, None] * nx[None] + np.abs(C0))).max() < 1e-13
+    L = pod._lib()
+    least = torch.empty(m * n * ((K + 65535) // 65536), dtype=torch.float64, device="cuda")
+    Xd, Yd, C = _dev(X), _dev(Y), torch.empty((m, n), dtype=torch.float64, device="cuda")
+    assert L.irom_gram(pod.GRAM_FP64, m, n, K, Xd.data_ptr(), K, Yd.data_ptr(), K, C.data_ptr(), n, 0,
+                       least.data_ptr(), least.numel() * 8, pod._s()) == 0
+    assert (np.abs(C.cpu().numpy() - X @ Y.T) / scale).max() < 1e-13
+
+
+@pytest.mark.parametrize("mode,bound", [(pod.GRAM_FP32X3, 1e-6), (pod.GRAM_BF16X3, 1e-4)])
+def test_projection_of_many_vectors_in_the_split_modes(mode, bound):
+    """Above 64 basis vectors the split products are used (below, FP64 in every mode): their error
+    against the FP64 projection is within the mode's bound and not that of FP64."""
+    rng = np.random.default_rng(4)
+    nm, nq, n, r = 3, 4, 5, 70
+    verts = mesh.hex_box(n, 0.05, rng)
+    b = H.basis_modified_a(nm, nq)
+    jac, df = H.geom_device("hex", _dev(verts), nq, b["z"], True)
+    terms = pod.helmholtz_affine_terms(nm, nq, n ** 3, b, jac, df)
+    V = _dev(rng.standard_normal((r, n ** 3 * nm ** 3)))
+    for op in terms.values():
+        exact = pod.galerkin_project(op, V)[0]
+        got = pod.galerkin_project(op, V, mode=mode)[0]
+        err = float((got - exact).norm() / exact.norm())
+        print(f"mode {mode}: {err:.1e}")
+        assert 1e-13 < err < bound
+
+
 @pytest.mark.parametrize("m,K", [(65, 5_000), (130, 40_000), (195, 20_011), (384, 50_000)])
 def test_gram_skips_tiles_outside_the_result(m, K):
     """Blocks cut by the edge of C or by the diagonal, one to a few K slices per block."""
