@@ -265,19 +265,6 @@ imf::DenseArgs dense_args(const imf_op op, bool transpose, const double *in, dou
     return a;
 }
 
-__global__ void fill_identity(int n, double *__restrict__ d)
-{
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < (long)n * n) d[i] = i / n == i % n ? 1.0 : 0.0;
-}
-
-// v[i] = val for i in [0, n), else 0 up to len
-__global__ void fill_range(long len, long lo, long hi, double val, double *__restrict__ d)
-{
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < len) d[i] = i >= lo && i < hi ? val : 0.0;
-}
-
 imf::PencilArgs pencil_args(const imf_op op, const double *in, double *out)
 {
     imf::PencilArgs a{};
@@ -344,65 +331,40 @@ bool dense_pays(const imf_op op, int tr, bool helm, bool from_modes)
 }
 
 // The element matrices of a collapsed-shape operator for the dense kernel, read off the
-// runtime-size kernel itself: applied to the identity with unit Jacobians, it gives the
-// matrix with all its vertex and edge corrections.  For Helmholtz the derivative factors are
-// chosen so that one metric term remains: rows e_a give K_aa; a single row e_a + e_b or
-// e_a - e_b gives K_aa + K_bb + (K_ab + K_ba) or the same with a minus sign.
+// runtime-size kernel itself: applied to unit vectors (dense_units), it gives the matrix with all
+// its vertex and edge corrections; one run from the modes serves both directions of a transform.
 // Taken by BwdTrans, IProduct and their transposes and by Helmholtz with one set of factors
-// per element and at most 128 modes, where dense_pays() (mf_routes.hpp).
+// per element and at most 128 modes, where dense_pays() (mf_routes.hpp).  Making the operator
+// costs one run of that kernel more: 45 -> 57 to 80 us, Helmholtz tetrahedra 8,9 187 and triangles
+// 8,16 168 (with a run for each term and direction 65 to 585 us).  The scratch is at most
+// 288 x 4 400 doubles.
 int build_dense(imf_op op)
 {
     const int M = (int)op->M, Q = (int)op->Q;
     const bool helm = op->kind == imf::kHelmholtz && !op->deformed;
     if (op->shape == imf::kSeg || !(helm || op->kind == imf::kBwdTrans || op->kind == imf::kIProduct))
         return IMF_OK;
-    const int D = op->dim, ng = helm ? 1 + D * (D + 1) / 2 : 1;
-    const bool coef_in = op->kind != imf::kIProduct;
+    const int D = helm ? op->dim : 0, ng = 1 + D * (D + 1) / 2;
+    bool from_modes[2] = {op->kind != imf::kIProduct, op->kind == imf::kIProduct};
     for (int tr = 0; tr < (helm ? 1 : 2); ++tr) {
-        const bool from_modes = coef_in != (tr == 1);
         op->dense[tr] = helm ? imf::dense_shape(M, M, ng)
-                             : imf::dense_shape(from_modes ? M : Q, from_modes ? Q : M, 1);
-        if (!dense_pays(op, tr, helm, from_modes)) op->dense[tr].nt = 0;
+                             : imf::dense_shape(from_modes[tr] ? M : Q, from_modes[tr] ? Q : M, 1);
+        if (!dense_pays(op, tr, helm, from_modes[tr])) op->dense[tr].nt = 0;
     }
     if (!op->dense[0].nt && !op->dense[1].nt) return IMF_OK;
-    const long n = helm ? M : std::max(M, Q), nd = helm ? (long)D * D * M : 0;
+    const long nu = (long)imf::dense_runs(D) * M;  // unit vectors
     double *work = nullptr;
-    hipError_t e = hipMalloc(&work, (size_t)(2 * n * n + n + nd) * sizeof(double));
-    double *eye = work, *mat = eye + n * n, *jac = mat + n * n, *df = jac + n;
-    auto grid = [](long len) { return (unsigned)((len + 255) / 256); };
-    if (e == hipSuccess) fill_range<<<grid(n), 256>>>(n, 0, n, 1.0, jac);
+    hipError_t e = hipMalloc(&work, (size_t)(nu * (M + (helm ? M : Q) + 1 + D * D)) * sizeof(double));
+    double *in = work, *runs = in + nu * M, *jac = runs + nu * (helm ? M : Q), *df = jac + nu;
+    if (e == hipSuccess) e = imf::dense_units(M, D, in, jac, df, nullptr);
+    if (e == hipSuccess)
+        e = launch_general(op, !from_modes[0], (int)nu, 0, 1.0, in, runs, jac, df, nullptr);
     for (int tr = 0; tr < 2 && e == hipSuccess; ++tr) {
         const imf::DenseShape &sh = op->dense[tr];
         if (!sh.nt) continue;
         e = hipMalloc(&op->d_dense[tr], sh.tab_len() * sizeof(double));
-        if (e != hipSuccess) break;
-        fill_identity<<<grid((long)sh.K * sh.K), 256>>>(sh.K, eye);
-        // one run of the general kernel on K unit inputs, packed into term g with factor c
-        auto term = [&](int g, double lambda, double c, bool add) {
-            e = launch_general(op, tr == 1, sh.K, 0, lambda, eye, mat, jac, df, nullptr);
-            if (e == hipSuccess) e = imf::dense_pack(sh, g, mat, c, add, op->d_dense[tr], nullptr);
-        };
-        // derivative factors with first row x e_a + y e_b
-        auto factors = [&](int a, double x, int b, double y) {
-            fill_range<<<grid(nd), 256>>>(nd, (long)a * M, (long)(a + 1) * M, x, df);
-            if (b != a) fill_range<<<grid(M), 256>>>(M, 0, M, y, df + (long)b * M);
-        };
-        if (!helm) {
-            term(0, 0.0, 1.0, false);
-            continue;
-        }
-        fill_range<<<grid(nd), 256>>>(nd, 0, 0, 0.0, df);
-        term(0, 1.0, 1.0, false);
-        for (int a = 0, g = 1; a < D; ++a)
-            for (int b = a; b < D && e == hipSuccess; ++b, ++g) {
-                factors(a, 1.0, b, 1.0);
-                term(g, 0.0, a == b ? 1.0 : 0.5, false);
-                if (a == b || e != hipSuccess) continue;
-                factors(a, 1.0, b, -1.0);
-                term(g, 0.0, -0.5, true);
-            }
+        if (e == hipSuccess) e = imf::dense_pack(sh, !from_modes[tr], runs, op->d_dense[tr], nullptr);
     }
-    if (e == hipSuccess) e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     (void)hipFree(work);
     if (e != hipSuccess) return hip_fail(e, "dense element matrices");

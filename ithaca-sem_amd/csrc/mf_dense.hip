@@ -146,20 +146,67 @@ __global__ __launch_bounds__(256) void dense_kernel(DenseArgs a)
     }
 }
 
-// One thread per entry of the fragment-ordered table of geometry term g:
+// Runs of a geometry term: the first, and for a pair of directions the one after it, of which
+// half the difference counts.
+__device__ __forceinline__ int first_run(int ng, int g, bool &pair)
+{
+    const int D = ng == 1 ? 0 : ng == 4 ? 2 : 3;
+    int r = 1;
+    pair = false;
+    if (g == 0) return 0;
+    for (int a = 0, h = 1; a < D; ++a)
+        for (int b = a; b < D; ++b, ++h) {
+            pair = b != a;
+            if (h == g) return r;
+            r += pair ? 2 : 1;
+        }
+    return r;
+}
+
+// One thread per entry of the fragment-ordered table, in its order:
 // [column group][step][g][tile][lane][2], lane = 16 kq + column, k = 8 step + 2 kq + component.
-__global__ void dense_pack_kernel(DenseShape sh, int g, const double *__restrict__ src, double c,
-                                  int add, double *__restrict__ tab)
+__global__ void dense_pack_kernel(DenseShape sh, int transposed, const double *__restrict__ runs,
+                                  double *__restrict__ tab)
 {
     const int steps = sh.kp / KSTEP, per = sh.nt * 128;
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)sh.ncg * steps * per) return;
-    const int w = (int)(i % per), step = (int)(i / per) % steps, cg = (int)(i / per / steps);
+    if (i >= (long)sh.ncg * steps * sh.ng * per) return;
+    const int w = (int)(i % per), g = (int)(i / per) % sh.ng, step = (int)(i / per / sh.ng) % steps,
+              cg = (int)(i / per / sh.ng / steps);
     const int comp = w & 1, lane = (w >> 1) & 63, t = w >> 7;
     const int k = step * KSTEP + 2 * (lane >> 4) + comp, n = (cg * sh.nt + t) * 16 + (lane & 15);
-    const double v = k < sh.K && n < sh.N ? c * src[(long)k * sh.N + n] : 0.0;
-    double *d = tab + ((long)(cg * steps + step) * sh.ng + g) * per + w;
-    *d = add ? *d + v : v;
+    double v = 0.0;
+    if (k < sh.K && n < sh.N) {
+        const long KN = (long)sh.K * sh.N;
+        bool pair;
+        const double *src = runs + first_run(sh.ng, g, pair) * KN +
+                            (transposed ? (long)n * sh.K + k : (long)k * sh.N + n);
+        v = pair ? 0.5 * (src[0] - src[KN]) : src[0];
+    }
+    tab[i] = v;
+}
+
+__global__ void dense_units_kernel(int M, int D, int nrun, double *__restrict__ in,
+                                   double *__restrict__ jac, double *__restrict__ df)
+{
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int n = nrun * M;  // elements
+    if (i >= (long)n * M) return;
+    const int e = (int)(i / M), m = (int)(i - (long)e * M), run = e / M;
+    in[i] = e - run * M == m ? 1.0 : 0.0;
+    if (m) return;
+    jac[e] = run ? 0x1p-200 : 1.0;
+    double f[3] = {0.0, 0.0, 0.0};
+    for (int a = 0, r = 1; a < D; ++a)
+        for (int b = a; b < D; ++b) {
+            if (r == run || (b != a && r + 1 == run)) {
+                f[a] = 0x1p100;
+                f[b] = r == run ? 0x1p100 : -0x1p100;
+            }
+            r += b != a ? 2 : 1;
+        }
+    for (int c = 0; c < D; ++c)
+        for (int d = 0; d < D; ++d) df[(long)(c * D + d) * n + e] = c == 0 ? f[d] : 0.0;
 }
 
 template <int NG>
@@ -200,11 +247,19 @@ DenseShape dense_shape(int K, int N, int ng)
     return sh;
 }
 
-hipError_t dense_pack(const DenseShape &sh, int g, const double *src, double c, bool add,
-                      double *tab, hipStream_t s)
+int dense_runs(int D) { return D == 0 ? 1 : D == 2 ? 5 : 10; }
+
+hipError_t dense_units(int M, int D, double *in, double *jac, double *df, hipStream_t s)
 {
-    const long n = (long)sh.ncg * (sh.kp / KSTEP) * sh.nt * 128;
-    dense_pack_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(sh, g, src, c, add ? 1 : 0, tab);
+    const long n = (long)dense_runs(D) * M * M;
+    dense_units_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(M, D, dense_runs(D), in, jac, df);
+    return hipGetLastError();
+}
+
+hipError_t dense_pack(const DenseShape &sh, bool transposed, const double *runs, double *tab, hipStream_t s)
+{
+    const long n = (long)sh.tab_len();
+    dense_pack_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(sh, transposed ? 1 : 0, runs, tab);
     return hipGetLastError();
 }
 

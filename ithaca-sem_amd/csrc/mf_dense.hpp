@@ -35,10 +35,19 @@ struct DenseArgs {
 // kernel does not take it.
 DenseShape dense_shape(int K, int N, int ng);
 
-// T_g (K x N row-major, device), g-th geometry term, into the fragment-ordered table.
-// c * src is added to the entries when add is set, stored otherwise.
-hipError_t dense_pack(const DenseShape &sh, int g, const double *src, double c, bool add,
-                      double *tab, hipStream_t s);
+// All terms into the fragment-ordered table, from the runs of dense_units (device): T_g row-major,
+// K x N, or N x K where `transposed` is set.
+hipError_t dense_pack(const DenseShape &sh, bool transposed, const double *runs, double *tab, hipStream_t s);
+
+// Inputs that make an element kernel give its matrix: runs of M unit vectors with a Jacobian and
+// (D > 0) D x D derivative factors per element.  Transforms: one run with unit Jacobians.
+// Helmholtz with lambda = 1: the mass matrix (J = 1, no factors), then one run for each diagonal
+// metric term and two for each pair.  A run's factors are one row, so that one metric term remains:
+// e_a gives K_aa, e_a + e_b and e_a - e_b give K_aa + K_bb + (K_ab + K_ba) and the same with a
+// minus sign.  They are 2^100 with J = 2^-200, which leaves the stiffness as it is and 2^-200 of
+// the mass matrix beside it.
+int dense_runs(int D);  // 1 for D = 0
+hipError_t dense_units(int M, int D, double *in, double *jac, double *df, hipStream_t s);
 
 hipError_t launch_dense(const DenseArgs &a, hipStream_t s);
 

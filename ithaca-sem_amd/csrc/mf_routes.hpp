@@ -69,7 +69,7 @@ inline bool dense_pays(const DenseCase &c)
     }
     const double s = c.point_scale ? 1.7 : 1.0;  // the Jacobian per point is read beside the input
     if (c.pencil) return (tet || M <= 80) && n >= (tet ? 130 : prism ? 500 : 250) * s * M;
-    const double few = prism ? Q * (10 + M / 3.0) : Q * (4 + M / 7.0), most = prism ? 6000 : 3500;
+    const double few = prism ? Q * (14 + M / 3.0) : Q * (4 + M / 7.0), most = prism ? 6000 : 3500;
     return Q <= 40 || n >= (few < most ? few : most) * s;
 }
 
