@@ -17,7 +17,7 @@ No reference counterpart: the reference has no derivative capability on this pat
 """
 import torch
 
-from . import MFError, _stream_ptr, lib as _lib, rom as _rom
+from . import MFError, Operator, _stream_ptr, lib as _lib, rom as _rom
 
 
 class ReducedSolve(torch.autograd.Function):
@@ -55,10 +55,11 @@ class BwdTransFn(torch.autograd.Function):
 _MISFIT_PARTS = 2048  # IMF_MISFIT_PARTS
 
 
-def _residual_and_misfit(u, f, jw):
+def _residual_and_misfit(u, f, jw, own=True):
     """r = u - f and 0.5 * sum(jw * r * r).  FP64 vectors of one length on one GPU take one pass
-    that overwrites u; anything else (FP32, a broadcast or strided f) goes through torch."""
-    if all(t.is_cuda and t.dtype == torch.float64 and t.device == u.device and t.shape == u.shape
+    that overwrites u, where the caller owns it; anything else (FP32, a broadcast or strided f)
+    goes through torch."""
+    if own and all(t.is_cuda and t.dtype == torch.float64 and t.device == u.device and t.shape == u.shape
            and t.is_contiguous() and not t.is_neg() for t in (u, f, jw)):
         part, loss = u.new_empty(_MISFIT_PARTS), u.new_empty(())
         if _lib().imf_misfit_device(u.numel(), u.data_ptr(), f.data_ptr(), jw.data_ptr(),
@@ -73,7 +74,8 @@ class L2Misfit(torch.autograd.Function):
     @staticmethod
     def forward(ctx, u_hat, f, bwd, ipr, jw):
         u = bwd.apply(u_hat.detach().contiguous())
-        r, loss = _residual_and_misfit(u, f.detach(), jw.detach())
+        # an Operator's result is new; what another object returns may be kept by it
+        r, loss = _residual_and_misfit(u, f.detach(), jw.detach(), isinstance(bwd, Operator))
         ctx.ipr = ipr
         ctx.save_for_backward(r, jw)
         return loss

@@ -240,3 +240,29 @@ def test_misfit_sizes_and_forms(n):
         r, loss = _residual_and_misfit(tu, tf, tw)
         assert loss.shape == () and np.array_equal(r.cpu().numpy(), u - f)
         assert abs(loss.item() - float(want)) <= 1e-13 * float(want)
+
+
+def test_misfit_leaves_the_buffers_of_other_transforms_alone():
+    """A transform that is not an Operator may return a tensor it keeps, or its argument: it stays as
+    it was, and misfit and gradient are those of the general path."""
+    class Kept:
+        def __init__(self, u):
+            self.u = u
+
+        def apply(self, u_hat):
+            return self.u
+
+    class Identity:
+        def apply(self, x):
+            return x
+
+    rng = np.random.default_rng(6)
+    u, f, w = (_dev(rng.uniform(0.5, 2, 500)) for _ in range(3))
+    for bwd, coef in ((Kept(u), torch.zeros(1, dtype=torch.float64, device="cuda")), (Identity(), u)):
+        before = u.clone()
+        x = coef.detach().requires_grad_(True)
+        loss = L2Misfit.apply(x, f, bwd, Identity(), w)
+        assert torch.equal(u, before)
+        assert abs(loss.item() - 0.5 * float((w * (u - f) ** 2).sum())) <= 1e-13 * loss.item()
+        if coef is u:
+            assert torch.equal(torch.autograd.grad(loss, x)[0], u - f)
