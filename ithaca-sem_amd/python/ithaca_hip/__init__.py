@@ -82,13 +82,18 @@ def _np_ptr(a):
     return a.ctypes.data_as(ctypes.c_void_p)
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_ptr(stream):
     """The hipStream_t of a torch stream, or of the current device's current stream.  The raw
-    handle of the current stream is asked for directly: torch.cuda.current_stream() builds a
-    Stream object, 2.6 us of a call whose launch takes 4."""
+    handle of the current stream is asked for directly where torch has the call (a private one):
+    torch.cuda.current_stream() builds a Stream object, 2.6 us of a call whose launch takes 4."""
     if stream is not None:
         return stream.cuda_stream
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    if _raw_stream is not None:
+        return _raw_stream(torch.cuda.current_device())
+    return torch.cuda.current_stream().cuda_stream
 
 
 def basis_modified_a(nm, nq):

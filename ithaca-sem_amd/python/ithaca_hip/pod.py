@@ -43,7 +43,7 @@ def _lib():
 
 
 def _s(stream=None):
-    return ctypes.c_void_p(_stream_ptr(stream))
+    return ctypes.c_void_p(_stream_ptr(stream or None))  # 0: the current stream
 
 
 def gram(X, Y=None, mode=GRAM_FP64, out=None, accumulate=False, work=None, stream=None,

@@ -51,7 +51,7 @@ def _ptr(t):
 
 
 def _stream(s):
-    return ctypes.c_void_p(_stream_ptr(s))
+    return ctypes.c_void_p(_stream_ptr(s or None))  # 0: the current stream
 
 
 class Batch:

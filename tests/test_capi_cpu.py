@@ -128,3 +128,22 @@ def test_gram_workspace_of_large_products_is_a_few_results():
     for m in (1, 12, 64, 65, 200, 2000):
         for K in (1, 1000, 65537, 10 ** 7):
             assert L.irom_gram_workspace_size(m, m, K) >= m * m * 8 * min(512, (K + 65535) // 65536)
+
+
+def test_stream_arguments(monkeypatch):
+    """None and (for the reduced-model calls) 0 mean the current stream; its handle is found through
+    the public call where torch lacks the direct one."""
+    import torch
+    import ithaca_hip as H
+    from ithaca_hip import pod, rom
+
+    class Stream:
+        cuda_stream = 77
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: Stream())
+    monkeypatch.setattr(H, "_raw_stream", lambda device: 1000 + device)
+    assert H._stream_ptr(None) == 1003 and H._stream_ptr(Stream()) == 77
+    for f in (pod._s, rom._stream):
+        assert f(None).value == f(0).value == 1003 and f(Stream()).value == 77
+    monkeypatch.setattr(H, "_raw_stream", None)
+    assert H._stream_ptr(None) == 77
