@@ -198,7 +198,7 @@ def rom_bench(args):
             st = status.cpu().numpy()
             r[name] = {"solves_per_s": n / (ms * 1e-3), "ms_per_batch": ms,
                        "frac_of_hbm_floor": r["hbm_floor_ms"] / ms,
-                       "variant": B.variants()[v],
+                       "variant": "the FP64 kernel" if method == rom.LU_FP64 else B.variants()[v],
                        "refinement_iters_max": int(iters.max()),
                        "refinement_iters_mean": float(iters.float().mean()),
                        "status_counts": np.bincount(st, minlength=4).tolist()}

@@ -1530,6 +1530,14 @@ int irom_batch_autotune(irom_batch b, int method, const double *d_A, const doubl
     if (!b || method < 0 || method > 2) return fail(1, "irom_batch_autotune: bad argument");
     const int slot = method != IROM_LU_FP64;
     hipStream_t s = (hipStream_t)stream;
+    if (method == IROM_LU_FP64) {  // one kernel: nothing to choose
+        if (int st = launch_solve(b, method, b->variant[slot], 0, d_A, d_theta, d_b, d_x, 1e-14, 10,
+                                  nullptr, nullptr, s))
+            return st;
+        IROM_CHECK(hipStreamSynchronize(s), "sync");
+        if (chosen) *chosen = b->variant[slot];
+        return 0;
+    }
     hipEvent_t e0, e1;
     IROM_CHECK(hipEventCreate(&e0), "event");
     IROM_CHECK(hipEventCreate(&e1), "event");

@@ -364,3 +364,13 @@ def test_fp64_solves_with_pivots_beyond_the_reciprocal(transpose):
         back = np.abs(b - Rs[i] @ y).max() / (np.abs(Rs[i]).sum(1).max() * np.abs(y).max() + np.abs(b).max())
         bar = 4 * max(n, 4) * 2.2e-16 + (n * 2.0 ** -24 if cases[i][1] == -1050 else 0.0)
         assert back < bar, (cases[i], back)
+
+
+def test_autotune_of_the_fp64_kernel_keeps_what_is_set(small):
+    bt, B = small
+    A, th, b = _dev(bt["A"]), _dev(bt["theta"]), _dev(bt["b"])
+    for v in (3, 0):
+        x = torch.zeros_like(b)
+        B.set_variant(rom.LU_FP64, v)
+        assert B.autotune(A, th, b, x, rom.LU_FP64) == v
+        assert _max_rel(bt, x.cpu().numpy(), R.solve(bt)) < TOL
