@@ -1260,7 +1260,8 @@ __global__ void reset_counters(int *c, int *d)
 // dJ/dmu_q = -lambda^T A_q x, one workgroup per instance and term: a lane owns the columns
 // lane + 64 s (its x in registers), a wave every fourth row, four rows' loads in flight.  With
 // one workgroup per instance and a thread walking down each column, 96 instances of up to 64
-// took 95 us.
+// took 95 us.  Instances of at most 16 rows take a wave per term, 16 columns by four rows at a time
+// (4 096 of 4 rows 17 us that first way, 22 with a workgroup per term, now 7).
 __global__ __launch_bounds__(NT) void param_grad_kernel(BatchDev bd, const double *__restrict__ A,
                                                         const double *__restrict__ lam,
                                                         const double *__restrict__ x,
@@ -1272,6 +1273,21 @@ __global__ __launch_bounds__(NT) void param_grad_kernel(BatchDev bd, const doubl
     const int n = bd.N[inst], nq = bd.Q[inst];
     if ((int)blockIdx.y >= nq) return;
     const long vo = bd.voff[inst];
+    if (n <= 16) {
+        if (blockIdx.y) return;
+        const int r = lane >> 4, j = lane & 15;
+        const double xj = j < n ? x[vo + j] : 0.0;
+        for (int q = w; q < nq; q += NW) {
+            const double *Aq = A + bd.aoff[inst] + (long)q * n * n;
+            double acc = 0.0;
+#pragma unroll
+            for (int i0 = 0; i0 < 16; i0 += 4)
+                if (i0 + r < n && j < n) acc = fma(lam[vo + i0 + r] * Aq[(i0 + r) * n + j], xj, acc);
+            acc = wave_sum(acc);
+            if (lane == 0) grad[bd.toff[inst] + q] = -acc;
+        }
+        return;
+    }
     if ((int)threadIdx.x < n) ls[threadIdx.x] = lam[vo + threadIdx.x];
     double xs[CS];
 #pragma unroll
@@ -1604,7 +1620,8 @@ int irom_batch_param_grad(irom_batch b, const double *d_A, const double *d_lambd
                           const double *d_x, double *d_grad, void *stream)
 {
     if (!b || !d_A || !d_lambda || !d_x || !d_grad) return fail(1, "irom_batch_param_grad: bad argument");
-    const dim3 grid((unsigned)b->nInst, (unsigned)std::min(b->qmax, 1024));
+    const int nmax = *std::max_element(b->N.begin(), b->N.end());
+    const dim3 grid((unsigned)b->nInst, (unsigned)(nmax <= 16 ? 1 : std::min(b->qmax, 1024)));
     irom::param_grad_kernel<<<grid, irom::NT, 0, (hipStream_t)stream>>>(dev_view(b), d_A, d_lambda,
                                                                         d_x, d_grad);
     IROM_CHECK(hipGetLastError(), "param_grad launch");

@@ -374,3 +374,21 @@ def test_autotune_of_the_fp64_kernel_keeps_what_is_set(small):
         B.set_variant(rom.LU_FP64, v)
         assert B.autotune(A, th, b, x, rom.LU_FP64) == v
         assert _max_rel(bt, x.cpu().numpy(), R.solve(bt)) < TOL
+
+
+def test_param_grad_of_small_systems():
+    """1 to 17 rows, 1 to 9 terms, where a wave takes a term; a batch of small ones alone and one
+    with a larger system.  Bar: n roundings of the terms' absolute sum."""
+    rng = np.random.default_rng(9)
+    for extra in ([], [17, 40]):
+        N = [1, 2, 3, 4, 5, 7, 8, 12, 15, 16] + extra
+        Q = [1 + (3 * i) % 9 for i in range(len(N))]
+        B = rom.Batch(N, Q)
+        A, lam, x = (rng.standard_normal(k) for k in (B.a_size, B.v_size, B.v_size))
+        got = B.param_grad(_dev(A), _dev(lam), _dev(x)).cpu().numpy()
+        for i, (n, nq) in enumerate(zip(N, Q)):
+            M = A[B.a_off[i]:B.a_off[i] + nq * n * n].reshape(nq, n, n)
+            lv, xv = lam[B.v_off[i]:B.v_off[i] + n], x[B.v_off[i]:B.v_off[i] + n]
+            for q in range(nq):
+                bar = 1e-15 * max(n, 4) * (np.abs(lv) @ np.abs(M[q]) @ np.abs(xv))
+                assert abs(got[B.t_off[i] + q] + lv @ M[q] @ xv) <= bar, (n, q)
