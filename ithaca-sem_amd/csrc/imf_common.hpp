@@ -10,6 +10,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <type_traits>
 
 namespace imf {
 
@@ -59,8 +60,8 @@ struct HexCfg {
     static constexpr int BLOCK = ((EPB * TPE + 63) / 64) * 64;
 };
 
-// The table argument, read where the kernel's arguments lie; for kernels whose first argument
-// it is.  Each call is a new place to the compiler, so a table used through it is loaded where
+// The table argument, read where the kernel's arguments lie: it must be the kernel's first
+// argument, which a launch checks with table_first.  Each call is a new place to the compiler, so a table used through it is loaded where
 // it is used.  Otherwise the compiler loads every table into scalar registers at the start and
 // moves what does not fit to lanes of vector registers (8 modes, 9 points: 670 values, two
 // moves back for each product), or, with a lane-dependent index and some 300 uses, copies the
@@ -68,6 +69,18 @@ struct HexCfg {
 // Helmholtz regular 8,9 2 056/108 and 7,8 95/86, deformed 8,9 258/180 and 7,8 152/136;
 // BwdTrans 8,9 70/39; quad Helmholtz regular 8,10 1 345/88.  AGAIN = false leaves the table to
 // the compiler, for kernels that it slows down.
+template <typename Kernel, typename TabT>
+struct TableFirst;
+template <typename First, typename... Rest, typename TabT>
+struct TableFirst<void (*)(First, Rest...), TabT> {
+    static constexpr bool value = std::is_same_v<First, TabT>;
+};
+template <typename TabT, typename Kernel>
+constexpr bool table_first(Kernel)
+{
+    return TableFirst<Kernel, TabT>::value;
+}
+
 template <bool AGAIN = true, typename TabT>
 __device__ __forceinline__ decltype(auto) reread(const TabT &tab)
 {

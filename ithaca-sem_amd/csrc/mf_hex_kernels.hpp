@@ -122,7 +122,7 @@ __device__ __forceinline__ void store_modes_block(T *__restrict__ dst, int nv, B
 
 // Mode pencils -> u (registers, k-column of thread (i,j)).  pencil(p) returns the p-th
 // coefficient of this thread's p-pencil (t = r*NM + q); uses buf0 and buf1.
-template <int NM, int NQ, typename T, bool AGAIN = true, typename PencilFn>
+template <int NM, int NQ, typename T, bool AGAIN, typename PencilFn>
 __device__ __forceinline__ void hex_bwd_to_columns(const Tab<NM, NQ, T> &tab, PencilFn pencil,
                                                    bool active, int t, T *buf0, T *buf1,
                                                    T (&u)[NQ])
@@ -180,7 +180,7 @@ __device__ __forceinline__ void hex_bwd_to_columns(const Tab<NM, NQ, T> &tab, Pe
 // k-columns acc (registers of thread (i,j)) -> (B x B x B)^T acc; emit(p, v) receives the
 // p-th coefficient of this thread's p-pencil (t = r*NM + q).  Uses buf0 and buf1; emit may
 // write to buf0.
-template <int NM, int NQ, typename T, bool AGAIN = true, typename EmitFn>
+template <int NM, int NQ, typename T, bool AGAIN, typename EmitFn>
 __device__ __forceinline__ void hex_columns_to_modes(const Tab<NM, NQ, T> &tab,
                                                      const T (&acc)[NQ], bool active, int t,
                                                      T *buf0, T *buf1, EmitFn emit)
@@ -263,7 +263,7 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_bwdtrans_kernel(
         for (int p = 0; p < NM; ++p) uh[p] = T(0);
     }
     T u[NQ];
-    hex_bwd_to_columns<NM, NQ, T>(tab, [&](int p) { return uh[p]; }, active, t, lds[es][0],
+    hex_bwd_to_columns<NM, NQ, T, true>(tab, [&](int p) { return uh[p]; }, active, t, lds[es][0],
                                   lds[es][1], u);
     if (!valid) return;
     if (DIR == kTranspose) {
@@ -481,7 +481,7 @@ __global__ __launch_bounds__((HexCfg<NQ, WIDE>::BLOCK)) void hex_helmholtz_kerne
         load_modes_block<NM, NQ, C, T>(in + e0 * M, nv, [&](int sl) { return lds[sl][2]; });
     __syncthreads();
     T u[NQ];
-    hex_bwd_to_columns<NM, NQ, T>(
+    hex_bwd_to_columns<NM, NQ, T, true>(
         tab, [&](int p) { return buf2[t * (NM + 1) + p]; }, active, t, buf0, buf1, u);
     // buf2 (the mode pencils) was last read before the first barrier above
     if (active) {
@@ -642,8 +642,8 @@ __global__ __launch_bounds__((HexCfg<NQ, WIDE>::BLOCK)) void hex_helmholtz_kerne
     }
 
     // 5. (B x B x B)^T of the combined quadrature-space field, then one coalesced store.
-    hex_columns_to_modes<NM, NQ, T>(tab, acc, active, t, buf0, buf1,
-                                    [&](int p, T v) { buf2[t * (NM + 1) + p] = v; });
+    hex_columns_to_modes<NM, NQ, T, true>(tab, acc, active, t, buf0, buf1,
+                                          [&](int p, T v) { buf2[t * (NM + 1) + p] = v; });
     __syncthreads();
     store_modes_block<NM, NQ, C, T>(out + e0 * M, nv, [&](int sl) { return lds[sl][2]; });
   }

@@ -36,6 +36,7 @@ hipError_t launch_hex(const LaunchArgs &a)
         auto launch = [&](auto wide) {
             constexpr bool WIDE = decltype(wide)::value;
             using W = HexCfg<NQ, WIDE>;
+            static_assert(table_first<Tab<NM, NQ, T>>(&hex_helmholtz_kernel<NM, NQ, T, GEO, WIDE>));
             const dim3 g((unsigned)((a.nElmt + W::EPB - 1) / W::EPB)), b(W::BLOCK);
             if constexpr (std::is_same_v<T, double>) {
                 if (a.gmap) {
@@ -56,6 +57,7 @@ hipError_t launch_hex(const LaunchArgs &a)
         }
         launch(std::false_type{});
     } else if constexpr (KIND == kMass) {
+        static_assert(table_first<Tab<NM, NQ, T>>(&hex_mass_kernel<NM, NQ, T, GEO>));
         hex_mass_kernel<NM, NQ, T, GEO><<<grid, block, 0, a.stream>>>(
             tab, a.nElmt, a.nvec, in, a.ldin, geom, out, a.ldout);
     } else if constexpr (KIND == kIProdDeriv) {
@@ -63,6 +65,7 @@ hipError_t launch_hex(const LaunchArgs &a)
             <<<grid, block, 0, a.stream>>>(tab, a.nElmt, in, geom, out);
     } else if constexpr ((KIND == kBwdTrans && DIR == kForward) ||
                          (KIND == kIProduct && DIR == kTranspose)) {
+        static_assert(table_first<Tab<NM, NQ, T>>(&hex_bwdtrans_kernel<NM, NQ, T, DIR, GEO>));
         hex_bwdtrans_kernel<NM, NQ, T, DIR, GEO>
             <<<grid, block, 0, a.stream>>>(tab, a.nElmt, in, geom, out);
     } else {
@@ -83,6 +86,7 @@ hipError_t launch_quad(const LaunchArgs &a)
     const T *geom = static_cast<const T *>(a.geom);
     T *out = static_cast<T *>(a.out);
     if constexpr (KIND == kHelmholtz) {
+        static_assert(table_first<Tab<NM, NQ, T>>(&quad_helmholtz_kernel<NM, NQ, T, GEO>));
         quad_helmholtz_kernel<NM, NQ, T, GEO>
             <<<grid, block, 0, a.stream>>>(tab, a.nElmt, T(a.lambda), in, geom, out, a.skip);
     } else if constexpr (KIND == kIProdDeriv) {
@@ -90,6 +94,7 @@ hipError_t launch_quad(const LaunchArgs &a)
             <<<grid, block, 0, a.stream>>>(tab, a.nElmt, in, geom, out);
     } else if constexpr ((KIND == kBwdTrans && DIR == kForward) ||
                          (KIND == kIProduct && DIR == kTranspose)) {
+        static_assert(table_first<Tab<NM, NQ, T>>(&quad_bwdtrans_kernel<NM, NQ, T, DIR, GEO>));
         quad_bwdtrans_kernel<NM, NQ, T, DIR, GEO>
             <<<grid, block, 0, a.stream>>>(tab, a.nElmt, in, geom, out);
     } else {

@@ -16,7 +16,7 @@
 namespace imf {
 
 // u_hat (global) -> u (registers: thread i holds u[j] at point (i, j)).  Uses buf0.
-template <int NM, int NQ, typename T, bool AGAIN = true>
+template <int NM, int NQ, typename T, bool AGAIN>
 __device__ __forceinline__ void quad_bwd_to_lines(const Tab<NM, NQ, T> &tab,
                                                   const T *__restrict__ src, bool valid,
                                                   bool active, int t, T *buf0, T (&u)[NQ])
@@ -60,7 +60,7 @@ __device__ __forceinline__ void quad_bwd_to_lines(const Tab<NM, NQ, T> &tab,
 
 // acc (registers, j-line of thread i) -> out = (B x B)^T acc.  Uses buf0; the caller
 // must have synchronised any earlier readers of buf0.
-template <int NM, int NQ, typename T, bool AGAIN = true>
+template <int NM, int NQ, typename T, bool AGAIN>
 __device__ __forceinline__ void quad_lines_to_modes(const Tab<NM, NQ, T> &tab,
                                                     const T (&acc)[NQ], T *__restrict__ dst,
                                                     bool valid, bool active, int t, T *buf0)
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(QuadCfg<NQ>::BLOCK) void quad_bwdtrans_kernel(
     const bool valid = active && e < nElmt;
 
     T u[NQ];
-    quad_bwd_to_lines<NM, NQ, T>(tab, in + e * M, valid, active, t, lds[es], u);
+    quad_bwd_to_lines<NM, NQ, T, true>(tab, in + e * M, valid, active, t, lds[es], u);
     if (!valid) return;
     if (DIR == kTranspose) {
         if (GEO == kDeformed) {
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(QuadCfg<NQ>::BLOCK) void quad_helmholtz_kernel(
         for (int j = 0; j < NQ; ++j) acc[j] += buf0[j * NQ + t];
     }
     __syncthreads();
-    quad_lines_to_modes<NM, NQ, T>(tab, acc, out + e * M, valid, active, t, buf1);
+    quad_lines_to_modes<NM, NQ, T, true>(tab, acc, out + e * M, valid, active, t, buf1);
 }
 
 // PhysDeriv, quads (PhysDeriv.h:260-400, PhysDerivKernels.hpp:93-137): out_0 = df0 d0 +
