@@ -459,11 +459,16 @@ __device__ __noinline__ void lu_panel_wave(GPtr A, GPtr E, int ld, int k0,
     };
     for_columns(column);
     if (zero && lane == 0) sh.zero = 1;
+    // lanes read what others left in LDS: the wave's accesses stay in order, the compiler's must too
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     put_pivots<64>(A, ld, k0, nb, ncol, lane);
     const unsigned long long below = (1ull << lane) - 1ull, left0 = __ballot(act0), left1 = __ballot(act1);
     if (act0) put_left(lane, __popcll(left0 & below), r0, A, ld, k0);
     if (TWO && act1) put_left(lane + 64, __popcll(left0) + __popcll(left1 & below), r1, A, ld, k0);
-    if constexpr (FULL) block_factors(E);
+    if constexpr (FULL) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        block_factors(E);
+    }
 }
 
 // The same for m > 128 rows (nb = 16) by the whole workgroup, one row per thread.  Per column
