@@ -466,7 +466,8 @@ def pod_bench(args):
           "symmetry_rel_err": (torch.linalg.matrix_norm(Ar - Ar.T)
                                / torch.linalg.matrix_norm(Ar)).item(),
           "bytes_per_launch_apply": E * 8 * (2 * M * r + 7 * Q),
-          "entry": "irom_galerkin_project (multi-vector apply + MFMA product)"}
+          "entry": "irom_galerkin_project (multi-vector apply + MFMA product)",
+          "split_modes": "products of at most 64 vectors are formed in FP64 in every mode"}
     for name in terms:
         ref = Cq[name].get("cpu")
         if ref is None:

@@ -412,7 +412,7 @@ struct DiagTab {
 // sum over the seven geometry terms of separable weights (B^2, dB^2 or B dB per direction), so
 // each term is contracted one direction at a time through LDS.  With one thread per mode
 // summing over all points it read the geometry once per mode (8 000 elements of 6 modes:
-// 2.5 ms; now 0.2 ms).
+// 2.5 ms; now 0.12 ms).
 __global__ __launch_bounds__(256) void helm_diag_hex(DiagTab t, int nm, int nq, int deformed,
                                                      double lambda,
                                                      const double *__restrict__ geom,

@@ -30,7 +30,8 @@ typedef dv2 dv2u __attribute__((aligned(8)));  // rows of A are 8-byte aligned
 
 constexpr int KSTEP = 8;  // k per pair of MFMA steps
 
-// steps per LDS chunk: as many as keep the chunk within 32 KB
+// steps per LDS chunk: four of one term (NT * 4 KB, at most 32 KB), one of several (NG * NT KB, at
+// most 56 KB: Helmholtz tetrahedra of 8 modes, two workgroups per CU)
 constexpr int chunk_steps(int ng) { return ng == 1 ? 4 : 1; }
 
 // NT column tiles, NG geometry terms.

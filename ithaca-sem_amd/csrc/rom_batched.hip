@@ -146,7 +146,7 @@ struct PivLds {
 //
 // What bounds a batch is the chain of an instance's columns and the traffic of the factor
 // between the workgroup and memory (768 workgroups hold 430 MB, beyond every cache), so the
-// steps of the chain are short, several workgroups share a CU (43 KB of LDS and at most 168
+// steps of the chain are short, several workgroups share a CU (47.6 KB of LDS and at most 168
 // VGPRs: three), and the matrix is passed over once:
 //   * left-looking: a panel of 16 columns is read once, brought up to date with all earlier
 //     panels while it sits in the accumulators of four waves, factored and written once; an
@@ -201,6 +201,7 @@ struct LuLds {
     int zero;                      // a pivot without a finite reciprocal (lu_divide: zero or NaN)
     int inst;
 };
+static_assert(3 * sizeof(LuLds) <= 160 * 1024, "three workgroups per CU");
 __shared__ LuLds sh;  // of solve_fp64_kernel and the functions it calls
 
 // The phases are functions of their own (inlined into one kernel they spill each other's

@@ -171,3 +171,31 @@ def test_making_an_operator_with_dense_tables_takes_little_longer(key, few):
     small, large = best(few), best(40000)
     print(f"{key}: {small * 1e6:.0f} us, with tables {large * 1e6:.0f} us")
     assert large < 3.5 * small
+
+
+@pytest.mark.parametrize("shape,nm,nq,E", [("tri", 4, 5, 130), ("tet", 4, 5, 70), ("tet", 7, 8, 70),
+                                           ("prism", 5, 6, 70), ("pyr", 6, 7, 70), ("hex", 5, 6, 4003),
+                                           ("hex", 6, 7, 70), ("hex", 8, 9, 1501), ("quad", 6, 7, 130)])
+@pytest.mark.parametrize("deformed", [False, True])
+def test_helmholtz_over_its_own_input(shape, nm, nq, E, deformed):
+    """An element's coefficients are all read before any of its results is written, in every kernel
+    that Helmholtz takes: out may be the input, bit for bit."""
+    rng = np.random.default_rng(E + nm)
+    R = {"hex": [[0, 0, 0], [1, 0, 0], [1, 1, 0], [0, 1, 0], [0, 0, 1], [1, 0, 1], [1, 1, 1], [0, 1, 1]],
+         "quad": [[0, 0], [1, 0], [1, 1], [0, 1]], **REG}[shape]
+    R = np.array(R, dtype=float)
+    jitter = 0.1 if deformed or shape in ("tri", "tet") else 0.0
+    verts = R[None] * rng.uniform(0.5, 2.0, (E, 1, 1)) + jitter * rng.uniform(-1, 1, (E,) + R.shape)
+    box = shape in ("hex", "quad")
+    o = H.Operator(f"Helmholtz_{shape.capitalize()}_{'Deformed' if deformed else 'Regular'}", nm, nq, E)
+    pts = nq if box else {"tri": (nq, nq - 1), "tet": (nq, nq - 1, nq - 1)}.get(shape, (nq, nq, nq - 1))
+    jac, df = H.geom_device(shape, torch.from_numpy(verts).cuda(), pts,
+                            H.basis_modified_a(nm, nq)["z"] if box else None, deformed)
+    o.set_jac(jac)
+    o.set_df(df)
+    o.set_lambda(2.0)
+    u = torch.from_numpy(rng.uniform(-1, 1, o.in_size)).cuda()
+    want = o.apply(u)
+    got = u.clone()
+    o.apply(got, out=got)
+    assert torch.equal(got, want)
