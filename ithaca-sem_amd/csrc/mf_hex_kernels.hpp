@@ -427,6 +427,10 @@ __global__ __launch_bounds__((HexCfg<NQ, WIDE>::BLOCK)) void hex_helmholtz_kerne
 {
     if (GATHER && skip && *skip) return;
     using C = HexCfg<NQ, WIDE>;
+    // Tables held / read again, us: FP64 4,5 deformed 4.8/5.2 at 100 elements and 29.5/30.9 at
+    // 20 000, regular 5.0/5.3 at 1 000, but regular 5,5 53.4/50.8 at 60 000; FP32 6,8 5.6/4.9 at
+    // one, 5 and 6 points the same (more points: reread()).
+    constexpr bool AGAIN = sizeof(T) == 4 ? NQ >= 7 : NQ >= 6 || (GEO == kRegular && NM >= 5);
     using Lb = HexLds<NM, NQ>;
     constexpr int M = Lb::M, Q = Lb::Q, TPE = C::TPE;
     constexpr long GS = geo_stride(7 * Q, sizeof(T));
@@ -481,7 +485,7 @@ __global__ __launch_bounds__((HexCfg<NQ, WIDE>::BLOCK)) void hex_helmholtz_kerne
         load_modes_block<NM, NQ, C, T>(in + e0 * M, nv, [&](int sl) { return lds[sl][2]; });
     __syncthreads();
     T u[NQ];
-    hex_bwd_to_columns<NM, NQ, T, true>(
+    hex_bwd_to_columns<NM, NQ, T, AGAIN>(
         tab, [&](int p) { return buf2[t * (NM + 1) + p]; }, active, t, buf0, buf1, u);
     // buf2 (the mode pencils) was last read before the first barrier above
     if (active) {
@@ -494,7 +498,7 @@ __global__ __launch_bounds__((HexCfg<NQ, WIDE>::BLOCK)) void hex_helmholtz_kerne
     // thread (j,k) = (t%NQ, t/NQ), d1 on j-pencils of thread (i,k) = (t%NQ, t/NQ),
     // d2 on this thread's k-column.
     if (active) {
-        const auto &tb = reread(tab);
+        const auto &tb = reread<AGAIN>(tab);
         T v[NQ];
         {
             const int pj = t % NQ, pk = t / NQ;
@@ -509,7 +513,7 @@ __global__ __launch_bounds__((HexCfg<NQ, WIDE>::BLOCK)) void hex_helmholtz_kerne
             }
         }
         {
-            const auto &tb = reread(tab);
+            const auto &tb = reread<AGAIN>(tab);
             const int pi = t % NQ, pk = t / NQ;
 #pragma unroll
             for (int l = 0; l < NQ; ++l) v[l] = buf2[(pk * NQ + l) * NQ + pi];
@@ -525,8 +529,8 @@ __global__ __launch_bounds__((HexCfg<NQ, WIDE>::BLOCK)) void hex_helmholtz_kerne
     __syncthreads();
 
     // 3. Pointwise metric contraction and mass term on this thread's column.
-    const T wij = GEO == kRegular ? reread(tab).w[ci] * reread(tab).w[cj] : T(0);
-    const auto &tb = reread(tab);
+    const T wij = GEO == kRegular ? reread<AGAIN>(tab).w[ci] * reread<AGAIN>(tab).w[cj] : T(0);
+    const auto &tb = reread<AGAIN>(tab);
     T g0[NQ], g1[NQ], g2[NQ], acc[NQ];
     if (valid) {
 #pragma unroll
@@ -594,7 +598,7 @@ __global__ __launch_bounds__((HexCfg<NQ, WIDE>::BLOCK)) void hex_helmholtz_kerne
         }
     }
     // D^T along k in registers.
-    const auto &td = reread(tab);
+    const auto &td = reread<AGAIN>(tab);
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
         T s = acc[k];
@@ -607,7 +611,7 @@ __global__ __launch_bounds__((HexCfg<NQ, WIDE>::BLOCK)) void hex_helmholtz_kerne
     // 4. D^T along i (pencils of thread (j,k)) into buf2, then D^T along j (pencils of
     // thread (i,k)) added to it: three buffers instead of four per element.
     if (active) {
-        const auto &tb = reread(tab);
+        const auto &tb = reread<AGAIN>(tab);
         T v[NQ];
         const int pj = t % NQ, pk = t / NQ;
 #pragma unroll
@@ -622,7 +626,7 @@ __global__ __launch_bounds__((HexCfg<NQ, WIDE>::BLOCK)) void hex_helmholtz_kerne
     }
     __syncthreads();
     if (active) {
-        const auto &tb = reread(tab);
+        const auto &tb = reread<AGAIN>(tab);
         T v[NQ];
         const int pi = t % NQ, pk = t / NQ;
 #pragma unroll
@@ -642,7 +646,7 @@ __global__ __launch_bounds__((HexCfg<NQ, WIDE>::BLOCK)) void hex_helmholtz_kerne
     }
 
     // 5. (B x B x B)^T of the combined quadrature-space field, then one coalesced store.
-    hex_columns_to_modes<NM, NQ, T, true>(tab, acc, active, t, buf0, buf1,
+    hex_columns_to_modes<NM, NQ, T, AGAIN>(tab, acc, active, t, buf0, buf1,
                                           [&](int p, T v) { buf2[t * (NM + 1) + p] = v; });
     __syncthreads();
     store_modes_block<NM, NQ, C, T>(out + e0 * M, nv, [&](int sl) { return lds[sl][2]; });

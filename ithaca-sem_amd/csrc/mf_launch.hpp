@@ -87,8 +87,15 @@ hipError_t launch_quad(const LaunchArgs &a)
     T *out = static_cast<T *>(a.out);
     if constexpr (KIND == kHelmholtz) {
         static_assert(table_first<Tab<NM, NQ, T>>(&quad_helmholtz_kernel<NM, NQ, T, GEO>));
+        if constexpr (std::is_same_v<T, double>) {
+            if (a.skip) {
+                quad_helmholtz_kernel<NM, NQ, T, GEO, true>
+                    <<<grid, block, 0, a.stream>>>(tab, a.nElmt, T(a.lambda), in, geom, out, a.skip);
+                return hipGetLastError();
+            }
+        }
         quad_helmholtz_kernel<NM, NQ, T, GEO>
-            <<<grid, block, 0, a.stream>>>(tab, a.nElmt, T(a.lambda), in, geom, out, a.skip);
+            <<<grid, block, 0, a.stream>>>(tab, a.nElmt, T(a.lambda), in, geom, out, nullptr);
     } else if constexpr (KIND == kIProdDeriv) {
         quad_iprod_deriv_kernel<NM, NQ, T, GEO>
             <<<grid, block, 0, a.stream>>>(tab, a.nElmt, in, geom, out);

@@ -159,17 +159,18 @@ __global__ __launch_bounds__(QuadCfg<NQ>::BLOCK) void quad_iproduct_kernel(
     quad_lines_to_modes<NM, NQ, T, false>(tab, acc, out + e * M, valid, active, t, lds[es]);
 }
 
-// skip (may be null) points to a device flag that makes the kernel return (an iteration queued past
-// the solver's last).  Packed geometry: deformed [e][4][Q] (Jw, JwG00, JwG01, JwG11); regular [e][4]
+// SKIP: skip points to a device flag that makes the kernel return (an iteration queued past the
+// solver's last); the test alone costs other applies up to 5 % (100 quads 8,9: 8.7 / 9.1 us).  Packed geometry: deformed [e][4][Q] (Jw, JwG00, JwG01, JwG11); regular [e][4]
 // (J, J G00, J G01, J G11) with the weights applied here.
-template <int NM, int NQ, typename T, int GEO>
+template <int NM, int NQ, typename T, int GEO, bool SKIP = false>
 __global__ __launch_bounds__(QuadCfg<NQ>::BLOCK) void quad_helmholtz_kernel(
     const Tab<NM, NQ, T> tab, int nElmt, T lambda, const T *__restrict__ in,
     const T *__restrict__ geom, T *__restrict__ out, const int *__restrict__ skip)
 {
-    if (skip && *skip) return;
+    if (SKIP && *skip) return;
     using C = QuadCfg<NQ>;
-    constexpr bool AGAIN = NQ >= 9;  // 6,8 deformed at 12e6 points: held 77 us, read again 80
+    // held / read again, us: 6,8 deformed at 12e6 points 77/80; FP32 regular 7,9 at 60 000 quads 17.4/18.1
+    constexpr bool AGAIN = NQ >= (sizeof(T) == 8 ? 9 : 10);
     constexpr int M = NM * NM, Q = NQ * NQ;
     __shared__ T lds[C::EPB][2][Q];
     const int eb = threadIdx.x / C::TPE;
