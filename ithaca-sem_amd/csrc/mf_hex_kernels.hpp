@@ -330,15 +330,18 @@ __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_iproduct_kernel(
 // of the reference's MassMatrixOp_MatFree (StdRegions/StdExpansion.cpp:647-661:
 // BwdTrans, then IProductWRTBase).  The thread's geometry column (NQ values of w J) is
 // read once and reused for every vector, so each further vector streams only its
-// coefficients in and out.  From 8 points the tables are read again (12e6 points, held /
-// read again: 8,9 132/78 us, 8,10 114/49, 6,8 43/29; 5,7 27/30, 4,6 26/28).
+// coefficients in and out.  From 8 points the table is read again where it has more entries than
+// there are scalar registers.  Held / read again, us at 30 000 elements: FP64 deformed 8,10
+// 267/146, 6,8 60/45, FP32 8,12 146/85; FP64 regular 8,8 148/164 (at 1 000 elements 0.64 of the
+// time, though), 7,7 75/94; with at most 91 registers (FP64 5,9, FP32 8,10 and 7,13) reading again
+// took 1.01 to 1.14 times as long.
 template <int NM, int NQ, typename T, int GEO>
 __global__ __launch_bounds__(HexCfg<NQ>::BLOCK) void hex_mass_kernel(
     const Tab<NM, NQ, T> tab, int nElmt, int nvec, const T *__restrict__ in, long ldin,
     const T *__restrict__ geom, T *__restrict__ out, long ldout)
 {
     using C = HexCfg<NQ>;
-    constexpr bool AGAIN = NQ >= 8;
+    constexpr bool AGAIN = NQ >= 8 && NM * NQ * (int)sizeof(T) / 4 > 95;
     constexpr int M = NM * NM * NM, Q = NQ * NQ * NQ;
     __shared__ T lds[C::EPB][2][Q];
     const int eb = threadIdx.x / C::TPE;
